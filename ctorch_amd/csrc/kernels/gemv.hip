@@ -1,11 +1,12 @@
 // Host dispatch of the projections: the GEMV (gemv_impl.h) for one or two activation rows (or shapes the matrix
 // cores do not take), the matrix-core kernel (gemm_rows.h) for a batch of decode rows, and the tiled matrix-core
-// kernel (gemm_tiles.h) for prefill chunks large enough to fill the device; all instantiated per epilogue in
-// gemv_*.hip.
+// kernel (gemm_tiles.h) for prefill chunks large enough to fill the device, and with f32 weights the f32 matrix-core
+// kernel (gemm_f32.h); all instantiated per epilogue in gemv_*.hip.
 //
 // The grid is persistent: one wave per row group, capped at the number of waves the chosen kernel keeps
 // resident on the device (its occupancy times the CU count), so every wave streams from the start and none
 // waits for another to retire.  LOGITS launches write one sampling candidate per work-group.
+#include "kernels/gemm_f32.h"
 #include "kernels/gemm_tiles.h"
 
 #include <mutex>
@@ -170,6 +171,25 @@ int launch_gemm(const dlk_gemv_params& params, hipStream_t stream) {
     return 0;
 }
 
+// f32 weights over several rows: one launch over all rows.
+int launch_f32(const dlk_gemv_params& p, hipStream_t stream) {
+    using namespace dlk::gemm32;
+    const int shape = shape_of(p);
+    const void* kernel = nullptr;
+    switch (p.epilogue) {
+    case DLK_EPI_STORE: kernel = dlk_gemm_f32_kernel_store(p, shape); break;
+    case DLK_EPI_RESIDUAL: kernel = dlk_gemm_f32_kernel_residual(p, shape); break;
+    case DLK_EPI_QKV: kernel = dlk_gemm_f32_kernel_qkv(p, shape); break;
+    case DLK_EPI_SWIGLU: kernel = dlk_gemm_f32_kernel_swiglu(p, shape); break;
+    default: break;
+    }
+    if (!kernel) return static_cast<int>(hipErrorInvalidValue);
+    const int64_t blocks = blocks_of(p, shape);
+    if (blocks > INT32_MAX) return static_cast<int>(hipErrorInvalidValue);
+    void* args[] = {const_cast<dlk_gemv_params*>(&p)};
+    return static_cast<int>(hipLaunchKernel(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kThreads), args, 0, stream));
+}
+
 // resident waves of a kernel on the current device (0 on error)
 int resident_waves(const Kernel& kernel) {
     static std::mutex mutex;
@@ -310,6 +330,7 @@ extern "C" int dlk_gemv(const dlk_gemv_params* params, dlh_stream stream_handle)
         return static_cast<int>(hipErrorInvalidValue);
     if (dlk::tiles::eligible(*params)) return launch_tiles(*params, stream);
     if (dlk::gemm::eligible(*params)) return launch_gemm(*params, stream);
+    if (dlk::gemm32::eligible(*params)) return launch_f32(*params, stream);
     const int waves = launch_waves(*params);
     if (waves <= 0) return static_cast<int>(hipErrorInvalidValue);
     const int blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;

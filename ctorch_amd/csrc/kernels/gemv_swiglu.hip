@@ -1,4 +1,5 @@
 // Projection kernels with the SWIGLU epilogue: the GEMV (one activation row) and the matrix-core variant.
+#include "kernels/gemm_f32.h"
 #include "kernels/gemm_tiles.h"
 
 dlk::gemv::Kernel dlk_gemv_kernel_swiglu(const dlk_gemv_params& p, int mt) {
@@ -15,4 +16,8 @@ dlk::gemv::Kernel dlk_gemm_reduce_swiglu(const dlk_gemv_params& p) {
 
 dlk::gemv::Kernel dlk_tiles_kernel_swiglu(const dlk_gemv_params& p) {
     return dlk::tiles::resolve<DLK_EPI_SWIGLU>(p);
+}
+
+const void* dlk_gemm_f32_kernel_swiglu(const dlk_gemv_params& p, int shape) {
+    return dlk::gemm32::resolve<DLK_EPI_SWIGLU>(p, shape);
 }
