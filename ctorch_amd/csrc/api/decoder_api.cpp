@@ -3,6 +3,7 @@
 #include "core/tensor_impl.h"
 #include "nn/decode_step.h"
 
+#include <algorithm>
 #include <cmath>
 
 #include <numeric>
@@ -102,9 +103,25 @@ dl_status dl_grouped_query_attention_noalloc(const float* query, const void* key
             throw std::invalid_argument("attention head size 2, 4, 8, 16, 32, 64 or 128");
         dlk_attention_params p{};
         p.kv_bf16 = kv_dtype == DL_BF16;
-        dl::detail::attention_split(batch, heads, kv_heads, D, p.kv_bf16 != 0, length, source, p.splits, p.chunk);
+        dl::detail::attention_split(batch, heads, kv_heads, D, p.kv_bf16 != 0, length, source, false, p.splits, p.chunk);
         const int64_t rows = batch * heads * length;
-        const int64_t need = p.splits > 1 ? rows * p.splits * (D + 2) : 0;
+        int64_t need = p.splits > 1 ? rows * p.splits * (D + 2) : 0;
+        if (length > 1) {
+            // several positions: the shapes that fit are those whose keys in 64-key tiles, split into up to
+            // 1024 / (B * KV) runs for two to four positions, do; the launch takes fewer splits where its own need more
+            const int64_t tiles = (source + 63) / 64, groups = batch * kv_heads;
+            const int64_t runs = length <= 4 ? std::min(tiles, (1024 + groups - 1) / groups) : 1;
+            const int64_t per = (tiles + runs - 1) / runs, most = (tiles + per - 1) / per;
+            if (most > 1 && rows * most * (D + 2) > DLK_ATTENTION_SCRATCH_FLOATS) {
+                need = rows * most * (D + 2);
+            } else {
+                while (need > DLK_ATTENTION_SCRATCH_FLOATS) {
+                    p.chunk *= 2;
+                    p.splits = static_cast<int>((source + p.chunk - 1) / p.chunk);
+                    need = p.splits > 1 ? rows * p.splits * (D + 2) : 0;
+                }
+            }
+        }
         if (need > DLK_ATTENTION_SCRATCH_FLOATS)
             throw std::invalid_argument("attention partials need " + std::to_string(need) +
                                         " floats, more than the allocation-free entry's " +

@@ -1,14 +1,28 @@
-// Split-K grouped-query decode attention (see dlk_attention_params in kernels.h).
+// Grouped-query attention over any number of query rows (see dlk_attention_params in kernels.h): one or several new
+// positions, causal or not, with or without a keep mask, head sizes 16 to 128.  (One position at head sizes 64 and 128
+// takes attention_matrix.hip, causal prefill chunks at those sizes attention_prefill.hip.)
 //
-// Grid (key split, query-row block, b * KV + kv head).  A work-group serves up to kRowsMax query rows of one
-// KV head: the H/KV query heads that share it, for one or more new positions.  It walks its key range in
-// tiles of T keys: the K and V tiles are loaded from HBM once (coalesced 16-byte loads, the next tile
-// prefetched into registers while the current one is used) and staged in LDS with a padded row stride, so
-// every query head of the group reuses them.  Scores use one lane per key, softmax is online (running max and
-// sum per row, wave64 reductions), P*V uses one lane per head-dim column.  With one split the work-group
-// writes the normalised output; otherwise it writes (o, max, sum) partials that attention_combine merges in a
-// second launch (the kernel boundary orders them: no device-scope fence, whose L2 write-back across the XCDs
-// costs microseconds per work-group).
+// All products run on the f32 matrix cores, so nothing is rounded that the inputs do not round: with
+// v_mfma_f32_16x16x4_f32, S^T[16 keys][16 rows] = K Q^T (lane l supplies K[key l%16] and Q[row l%16] at four consecutive
+// head-dim entries, 4 (l/16) .. +4 of each 16, one per product) and O^T[16 d][16 rows] += V^T P^T.  The scores come out
+// with lane l holding keys 4 (l/16) .. +4 of row l%16, which is the B operand of the second product when its k slot
+// l/16 of product j stands for key 4 (l/16) + j, so the probabilities never leave their lane; maximum, sum and rescale
+// factor of a row sit in the lanes of its column.
+//
+// Grid (key split, query-row block, b * KV + kv head).  The G query heads of a KV head at every new position are its
+// rows, position-major.  A work-group of four waves serves 16 WR of them: WR waves take 16 rows each, and the 4 / WR
+// waves of a row tile share the keys of each staged tile (merged in LDS at the end), so that a few rows still use all
+// four.  Key tiles are loaded with 16-byte loads (the next tile in flight, in registers, while one is used) and staged in
+// LDS as f32.  With one split the work-group writes the normalised output; otherwise it writes (o, max, sum) partials
+// that attention_combine merges in a second launch (the kernel boundary orders them: no device-scope fence, whose L2
+// write-back across the XCDs costs microseconds per work-group).
+//
+// What bounds it: many rows, the f32 matrix cores (153 TFLOP/s); few rows, the round trips of the K/V tiles.
+// Measured on MI355X (the kernel before it ran the products on the vector ALU, one key or head-dim column per lane):
+// 4 sequences x 7 positions over 1508 f32 keys, 32 / 8 heads of 64: 135.5 -> 11.6 us + 4.7 for the merge; 4 x 500
+// positions bidirectional over a padded batch: 455 -> 107 us (the products alone take 38; exponentials, masks and staging
+// as much vector work again, and the two barriers of a tile keep them from overlapping fully); causal byte prompts of
+// 4 x 510 positions, 8 / 2 heads of 32: 84 -> 18 us; one position of that model over 160 keys: 5.7 -> 5.1 us.
 #include "kernels/device_common.h"
 
 #include <algorithm>
@@ -20,186 +34,297 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kRowsMax = 16;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_any __attribute__((aligned(4))); // callers' rows: any float alignment
+typedef uint32_t u32_any __attribute__((aligned(1)));  // four mask bytes
 
-template <typename KT> struct KvTraits;
-template <> struct KvTraits<uint16_t> {
-    __device__ static __forceinline__ float at(const uint32_t* row, int d) {
-        const uint32_t w = row[d >> 1];
-        return (d & 1) ? bf16_hi(w) : bf16_lo(w);
-    }
-};
-template <> struct KvTraits<float> {
-    __device__ static __forceinline__ float at(const uint32_t* row, int d) { return __uint_as_float(row[d]); }
-};
+/// Keys per staged tile: few rows over small heads are a chain of tile round trips, so they take longer tiles.
+constexpr int tile_keys(int hd, int wr) { return hd == 16 || (hd == 32 && wr < 4) ? 128 : 64; }
 
-template <typename KT, int HD, int T>
-__global__ __launch_bounds__(kThreads) void attention_kernel(const dlk_attention_params p) {
-    constexpr int ES = sizeof(KT);
-    constexpr int ROW_WORDS = HD * ES / 4 + 1;            // padded LDS row: odd word stride, no bank conflicts
-    constexpr int CHUNKS_PER_ROW = HD * ES / 16;          // 16-byte chunks per K/V row
-    constexpr int TILE_CHUNKS = T * CHUNKS_PER_ROW;
-    constexpr int LOADS = (TILE_CHUNKS + kThreads - 1) / kThreads;
-    constexpr int DCOLS = (HD + kWave - 1) / kWave;       // head-dim columns per lane in P*V
-    constexpr int RPW = kRowsMax / kWaves;                // rows per wave
+// work-group barrier that orders LDS traffic only: the next tile's loads stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
-    __shared__ uint32_t k_tile[T * ROW_WORDS];
-    __shared__ uint32_t v_tile[T * ROW_WORDS];
-    __shared__ float q_tile[kRowsMax][HD];
-    __shared__ float p_tile[kRowsMax][T];
+template <typename KT, int HD, int WR>
+__global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_params p) {
+    constexpr int WK = kWaves / WR;                   // waves that share a row tile's keys
+    constexpr int T = tile_keys(HD, WR);
+    constexpr int GROUPS = T / 16 / WK;               // 16-key groups of a tile per wave
+    constexpr int KS = HD + 8, VS = HD + 4;           // LDS row strides (floats): conflict-free fragment reads
+    constexpr int VALUES = 16 / sizeof(KT);           // K/V values per 16-byte piece
+    constexpr int PIECES = HD / VALUES;               // pieces per K/V row
+    constexpr int LOADS = T * PIECES / kThreads;
+    constexpr int DT = HD / 16;                       // 16-wide head-dim tiles
+    static_assert(T % (16 * WK) == 0 && T * PIECES % kThreads == 0, "tile");
+    __shared__ __attribute__((aligned(16))) float k_tile[T][KS];
+    __shared__ __attribute__((aligned(16))) float v_tile[T][VS];
+    __shared__ int odd_values[kWaves]; // masked launches: whether the tile's V holds an infinity or NaN
 
-    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
-    const int split = blockIdx.x, row_block = blockIdx.y;
-    const int b = blockIdx.z / p.KV, kvh = blockIdx.z % p.KV;
+    const int t = threadIdx.x, lane = t % kWave, q = lane / 16, r = lane % 16;
+    const int wave = __builtin_amdgcn_readfirstlane(t / kWave), wr = wave / WK, wk = wave % WK;
+    // consecutive work-group ids go to the 8 XCDs in turn: each XCD takes a run of the order in which the splits and
+    // row blocks of a KV head are neighbours, so its L2 holds the few KV heads it works on
+    const int total = gridDim.x * gridDim.y * gridDim.z;
+    const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int xcd = id % 8, per = total / 8, rem = total % 8;
+    const int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + id / 8;
+    const int split = logical % gridDim.x, row_block = logical / gridDim.x % gridDim.y;
+    const int pair = logical / (gridDim.x * gridDim.y);
+    const int b = pair / p.KV, kvh = pair % p.KV;
     const int G = p.H / p.KV;
-    const int rows_total = G * p.L;
-    const int row0 = row_block * kRowsMax;
-    const int rows = min(kRowsMax, rows_total - row0);
-    const int64_t first = p.position ? *p.position : p.first_host;
-    const int64_t S = first + p.L;
+    const int rows_total = G * p.L, row0 = row_block * 16 * WR;
 
-    // query row r of this block -> (l, g): rows are ordered l-major so a block spans few positions
-    auto row_l = [&](int r) { return (row0 + r) / G; };
-    auto row_h = [&](int r) { return kvh * G + (row0 + r) % G; };
-
-    int64_t k_begin = static_cast<int64_t>(split) * p.chunk;
-    int64_t k_end = min(S, k_begin + p.chunk);
-    if (p.causal) k_end = min(k_end, first + row_l(rows - 1) + 1);
-
-    const size_t head_base = (static_cast<size_t>(b) * p.KV + kvh) * p.capacity;
+    const size_t head_base = static_cast<size_t>(pair) * p.capacity;
     const KT* kbase = static_cast<const KT*>(p.k) + head_base * HD;
     const KT* vbase = static_cast<const KT*>(p.v) + head_base * HD;
+    const int64_t k_begin = static_cast<int64_t>(split) * p.chunk;
 
-    // q rows (scaled once) into LDS
-    for (int i = t; i < rows * HD; i += kThreads) {
-        const int r = i / HD, d = i % HD;
-        const int64_t m = static_cast<int64_t>(b) * p.L + row_l(r);
-        q_tile[r][d] = p.q[m * p.ldq + static_cast<int64_t>(row_h(r)) * HD + d] * p.scale;
-    }
-
-    float m_run[RPW], l_run[RPW], o_acc[RPW][DCOLS];
-#pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-        m_run[j] = -INFINITY;
-        l_run[j] = 0.0f;
-#pragma unroll
-        for (int c = 0; c < DCOLS; ++c) o_acc[j][c] = 0.0f;
-    }
+    const int64_t first = p.position ? *p.position : p.first_host;
+    // this lane's query row (rows past the end repeat the last; their results are never written)
+    const int row = min(row0 + 16 * wr + r, rows_total - 1);
+    const int l = row / G, h = kvh * G + row % G;
+    const unsigned char* keep =
+        p.keep_mask ? p.keep_mask + b * p.mask_stride[0] + h * p.mask_stride[1] + l * p.mask_stride[2] : nullptr;
 
     u32x4 k_next[LOADS], v_next[LOADS];
-    auto load_tile = [&](int64_t tile0) {
+    uint32_t keep_next[GROUPS]; // four mask bytes each
+    // loads the tile's rows and this lane's mask entries; those from `end` on repeat the one before it and are dropped
+    // when the tile is used (the mask comes first: loads complete in order, and it would wait for the rows)
+    auto load_tile = [&](int64_t tile0, int64_t end) {
+        const int last = static_cast<int>(min<int64_t>(end - tile0, T)) - 1; // of the tile, uniform
+        if (keep) {
+            const int64_t stride = p.mask_stride[3];
+            const unsigned char* entries = keep + tile0 * stride;
+            if (stride == 1 && last == T - 1) {
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            const int chunk = t + i * kThreads;
-            const int key = chunk / CHUNKS_PER_ROW, part = chunk % CHUNKS_PER_ROW;
-            const int64_t kk = tile0 + key;
-            if (chunk < TILE_CHUNKS && kk < k_end) {
-                const size_t offset = static_cast<size_t>(kk) * HD * ES + static_cast<size_t>(part) * 16;
-                k_next[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(kbase) + offset);
-                v_next[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(vbase) + offset);
+                for (int g = 0; g < GROUPS; ++g)
+                    keep_next[g] = *reinterpret_cast<const u32_any*>(entries + 16 * (wk + WK * g) + 4 * q);
             } else {
-                k_next[i] = u32x4{0u, 0u, 0u, 0u};
-                v_next[i] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int g = 0; g < GROUPS; ++g) {
+                    uint32_t four = 0;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        four |= static_cast<uint32_t>(entries[min(16 * (wk + WK * g) + 4 * q + j, last) * stride]) << (8 * j);
+                    keep_next[g] = four;
+                }
             }
         }
-    };
-    auto store_tile = [&]() {
+        const KT* kt = kbase + tile0 * HD;
+        const KT* vt = vbase + tile0 * HD;
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) {
-            const int chunk = t + i * kThreads;
-            if (chunk < TILE_CHUNKS) {
-                const int key = chunk / CHUNKS_PER_ROW, part = chunk % CHUNKS_PER_ROW;
-                uint32_t* kd = k_tile + key * ROW_WORDS + part * 4;
-                uint32_t* vd = v_tile + key * ROW_WORDS + part * 4;
-                kd[0] = k_next[i].x; kd[1] = k_next[i].y; kd[2] = k_next[i].z; kd[3] = k_next[i].w;
-                vd[0] = v_next[i].x; vd[1] = v_next[i].y; vd[2] = v_next[i].z; vd[3] = v_next[i].w;
+            const int at = t + i * kThreads;
+            const uint32_t offset = min(at / PIECES, last) * HD + at % PIECES * VALUES;
+            k_next[i] = *reinterpret_cast<const u32x4*>(kt + offset);
+            v_next[i] = *reinterpret_cast<const u32x4*>(vt + offset);
+        }
+    };
+    // the first tile is requested before the device length arrives, within the storage: what lies past the length is
+    // dropped
+    const int64_t stored = min(p.capacity, k_begin + p.chunk);
+    if (k_begin < stored) load_tile(k_begin, stored);
+
+    const int64_t m_row = static_cast<int64_t>(b) * p.L + l;
+    f32x4 qf[DT];
+#pragma unroll
+    for (int s = 0; s < DT; ++s) {
+        const float* src = p.q + (p.q_row ? b * p.q_batch + l * p.q_row + h * p.q_head
+                                          : m_row * p.ldq + static_cast<int64_t>(h) * HD) + 16 * s + 4 * q;
+        qf[s] = *reinterpret_cast<const f32x4_any*>(src) * (p.scale * 1.4426950408889634f); // scores in base 2
+    }
+    // keys this lane's row sees, its wave's first and last row (wave_full: without a mask, every row of the wave sees
+    // the keys below it), and the work-group's last row
+    const int64_t S = first + p.L;
+    const int64_t split_end = min(S, k_begin + p.chunk);
+    const int64_t limit = p.causal ? min(split_end, first + l + 1) : split_end;
+    const int first_row = min(row0 + 16 * wr, rows_total - 1);
+    const int last_row = min(row0 + 16 * wr + 15, rows_total - 1), last_block_row = min(row0 + 16 * WR - 1, rows_total - 1);
+    const int64_t wave_full = p.causal ? min(split_end, first + first_row / G + 1) : split_end;
+    const int64_t wave_end = row0 + 16 * wr >= rows_total ? 0 // no row for this wave
+                             : p.causal                   ? min(split_end, first + last_row / G + 1)
+                                                          : split_end;
+    const int64_t k_end = p.causal ? min(split_end, first + last_block_row / G + 1) : split_end;
+
+    auto stage_tile = [&](int64_t tile0) {
+        const int staged = static_cast<int>(min<int64_t>(k_end - tile0, T)); // live keys of the tile
+        if (keep) {
+            bool odd = false;
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    odd |= (v_next[i][e] & 0x7f800000u) == 0x7f800000u;
+                    if constexpr (sizeof(KT) == 2) odd |= (v_next[i][e] & 0x7f80u) == 0x7f80u;
+                }
+            const bool any = __ballot(odd) != 0;
+            if (lane == 0) odd_values[wave] = any;
+        }
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int at = t + i * kThreads, key = at / PIECES, d = at % PIECES * VALUES;
+            const bool live = key < staged;
+            const u32x4 zero = {0u, 0u, 0u, 0u};
+            const u32x4 kv = live ? k_next[i] : zero, vv = live ? v_next[i] : zero;
+            if constexpr (sizeof(KT) == 4) {
+                *reinterpret_cast<u32x4*>(&k_tile[key][d]) = kv;
+                *reinterpret_cast<u32x4*>(&v_tile[key][d]) = vv;
+            } else {
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    const uint32_t k0 = half ? kv.z : kv.x, k1 = half ? kv.w : kv.y;
+                    const uint32_t v0 = half ? vv.z : vv.x, v1 = half ? vv.w : vv.y;
+                    *reinterpret_cast<f32x4*>(&k_tile[key][d + 4 * half]) = f32x4{bf16_lo(k0), bf16_hi(k0), bf16_lo(k1), bf16_hi(k1)};
+                    *reinterpret_cast<f32x4*>(&v_tile[key][d + 4 * half]) = f32x4{bf16_lo(v0), bf16_hi(v0), bf16_lo(v1), bf16_hi(v1)};
+                }
             }
         }
     };
 
-    if (k_begin < k_end) load_tile(k_begin);
-    for (int64_t tile0 = k_begin; tile0 < k_end; tile0 += T) {
-        __syncthreads(); // previous tile fully consumed (and q_tile written before the first tile)
-        store_tile();
-        __syncthreads();
-        if (tile0 + T < k_end) load_tile(tile0 + T); // in flight while this tile is used
+    float m_run = -INFINITY, l_run = 0.0f; // l_run: this lane's keys only
+    f32x4 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    for (int64_t tile0 = k_begin; tile0 < k_end; tile0 += T) {
+        lds_barrier(); // every wave is done with the previous tile
+        stage_tile(tile0);
+        // Tiles that reach past some row's keys, or have a mask: which of this lane's keys its row sees, four bits per
+        // group
+        uint32_t live = 0xffffffffu;
+        const bool partial = keep || tile0 + T > wave_full;
+        if (partial) {
+            const int rem = static_cast<int>(min<int64_t>(limit - tile0, T)); // keys of the tile below the limit
+            live = 0;
 #pragma unroll
-        for (int j = 0; j < RPW; ++j) {
-            const int r = wave + j * kWaves;
-            if (r >= rows) break;
-            // scores: lane = key
-            float s = -INFINITY;
-            const int64_t kk = tile0 + lane;
-            int64_t limit = k_end;
-            if (p.causal) limit = min(limit, first + row_l(r) + 1);
-            if (lane < T && kk < limit) {
-                const uint32_t* krow = k_tile + lane * ROW_WORDS;
-                float acc = 0.0f;
+            for (int g = 0; g < GROUPS; ++g) {
+                uint32_t four = (1u << min(max(rem - 16 * (wk + WK * g) - 4 * q, 0), 4)) - 1;
+                if (keep) {
 #pragma unroll
-                for (int d = 0; d < HD; ++d) acc += q_tile[r][d] * KvTraits<KT>::at(krow, d);
-                s = acc;
-                if (p.keep_mask && !p.keep_mask[b * p.mask_stride[0] + row_h(r) * p.mask_stride[1] +
-                                                row_l(r) * p.mask_stride[2] + kk * p.mask_stride[3]])
-                    s = -INFINITY;
-            }
-            const float tile_max = wave_max(s);
-            const float m_new = fmaxf(m_run[j], tile_max);
-            float pr = 0.0f, alpha = 1.0f;
-            if (m_new != -INFINITY) {
-                pr = s == -INFINITY ? 0.0f : expf(s - m_new);
-                alpha = m_run[j] == -INFINITY ? 0.0f : expf(m_run[j] - m_new);
-            }
-            const float tile_sum = wave_sum(pr);
-            l_run[j] = l_run[j] * alpha + tile_sum;
-            m_run[j] = m_new;
-            if (lane < T) p_tile[r][lane] = pr;
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            // P*V: lane = head-dim column
-#pragma unroll
-            for (int c = 0; c < DCOLS; ++c) {
-                const int d = lane + c * kWave;
-                float acc = o_acc[j][c] * alpha;
-                if (d < HD) {
-#pragma unroll 8
-                    for (int key = 0; key < T; ++key)
-                        acc += p_tile[r][key] * KvTraits<KT>::at(v_tile + key * ROW_WORDS, d);
+                    for (int j = 0; j < 4; ++j)
+                        if (!(keep_next[g] & (0xffu << (8 * j)))) four &= ~(1u << j);
                 }
-                o_acc[j][c] = acc;
+                live |= four << (4 * g);
             }
+        }
+        lds_barrier();
+        if (tile0 + T < k_end) load_tile(tile0 + T, k_end);
+        // nothing for this wave: its rows end before the tile, or the mask drops every key of its groups (whose zero
+        // probabilities still carry an infinity or NaN of V into the sums, as the reference's product does)
+        if (tile0 >= wave_end) continue;
+        if (partial && __ballot(live != 0) == 0 &&
+            !(keep && (odd_values[0] | odd_values[1] | odd_values[2] | odd_values[3])))
+            continue;
+
+        f32x4 s[GROUPS];
+        float tile_max = -INFINITY;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) s[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int d = 0; d < DT; ++d) {
+            f32x4 a[GROUPS];
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g)
+                a[g] = *reinterpret_cast<const f32x4*>(&k_tile[16 * (wk + WK * g) + r][16 * d + 4 * q]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int g = 0; g < GROUPS; ++g)
+                    s[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[g][e], qf[d][e], s[g], 0, 0, 0);
+        }
+        if (partial) {
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (!(live >> (4 * g + j) & 1)) s[g][j] = -INFINITY;
+        }
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) tile_max = fmaxf(tile_max, s[g][j]);
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, kWave));
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, kWave));
+        const float m_new = fmaxf(m_run, tile_max);
+        // a row that has seen no key yet keeps -inf, and nothing of its sums
+        const float m_safe = m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_safe);
+        l_run *= alpha;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o[d] *= alpha;
+        m_run = m_new;
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float e = __builtin_amdgcn_exp2f(s[g][j] - m_safe); // 0 for the dropped keys
+                s[g][j] = e;
+                l_run += e;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int d = 0; d < DT; ++d)
+                    o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_tile[16 * (wk + WK * g) + 4 * q + j][16 * d + r], s[g][j],
+                                                                o[d], 0, 0, 0);
         }
     }
+    l_run += __shfl_xor(l_run, 16, kWave);
+    l_run += __shfl_xor(l_run, 32, kWave);
 
-    // write results: the normalised output with one split, else (o, max, sum) partials for the combine pass
+    if constexpr (WK > 1) {
+        // merge the waves of a row tile, in wave order
+        constexpr int FLOATS = 4 * DT + 2; // per lane
+        static_assert(WR * (WK - 1) * FLOATS * kWave <= T * KS, "merge");
+        float* part = &k_tile[0][0];
+        lds_barrier();
+        if (wk > 0) {
+            float* mine = part + (wr * (WK - 1) + wk - 1) * FLOATS * kWave + lane;
 #pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-        const int r = wave + j * kWaves;
-        if (r >= rows) break;
-        const int l = row_l(r), h = row_h(r);
-        const int64_t m = static_cast<int64_t>(b) * p.L + l;
-        if (p.splits == 1) {
-            // a masked row that kept no key: NaN, as the reference's softmax over an all -inf row
-            const float inv = l_run[j] > 0.0f ? 1.0f / l_run[j] : p.keep_mask ? __builtin_nanf("") : 0.0f;
+            for (int i = 0; i < 4 * DT; ++i) mine[i * kWave] = o[i / 4][i % 4];
+            mine[4 * DT * kWave] = m_run;
+            mine[(4 * DT + 1) * kWave] = l_run;
+        }
+        lds_barrier();
+        if (wk > 0) return;
+        float mx = m_run;
 #pragma unroll
-            for (int c = 0; c < DCOLS; ++c) {
-                const int d = lane + c * kWave;
-                if (d < HD) p.out[m * p.ldo + static_cast<int64_t>(h) * HD + d] = o_acc[j][c] * inv;
-            }
-        } else {
-            const int64_t prow = (static_cast<int64_t>(b) * p.H + h) * p.L + l;
-            const int64_t slot = prow * p.splits + split;
+        for (int w = 0; w < WK - 1; ++w) mx = fmaxf(mx, part[((wr * (WK - 1) + w) * FLOATS + 4 * DT) * kWave + lane]);
+        const float safe = mx == -INFINITY ? 0.0f : mx;
+        const float own = __builtin_amdgcn_exp2f(m_run - safe);
+        l_run *= own;
 #pragma unroll
-            for (int c = 0; c < DCOLS; ++c) {
-                const int d = lane + c * kWave;
-                if (d < HD) p.partial_o[slot * HD + d] = o_acc[j][c];
-            }
-            if (lane == 0) {
-                p.partial_ml[slot * 2] = m_run[j];
-                p.partial_ml[slot * 2 + 1] = l_run[j];
-            }
+        for (int d = 0; d < DT; ++d) o[d] *= own;
+#pragma unroll
+        for (int w = 0; w < WK - 1; ++w) {
+            const float* theirs = part + (wr * (WK - 1) + w) * FLOATS * kWave + lane;
+            const float mw = theirs[4 * DT * kWave];
+            const float f = __builtin_amdgcn_exp2f(mw - safe);
+            l_run += f * theirs[(4 * DT + 1) * kWave];
+#pragma unroll
+            for (int i = 0; i < 4 * DT; ++i) o[i / 4][i % 4] += f * theirs[i * kWave];
+        }
+        m_run = mx;
+    }
+
+    if (row0 + 16 * wr + r >= rows_total) return;
+    if (p.splits == 1) {
+        // a masked row that kept no key: NaN, as the reference's softmax over an all -inf row
+        const float inv = l_run > 0.0f ? 1.0f / l_run : p.keep_mask ? __builtin_nanf("") : 0.0f;
+        float* out = p.out + m_row * p.ldo + static_cast<int64_t>(h) * HD + 4 * q;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_any*>(out + 16 * d) = o[d] * inv;
+    } else {
+        const int64_t slot = ((static_cast<int64_t>(b) * p.H + h) * p.L + l) * p.splits + split;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_any*>(p.partial_o + slot * HD + 16 * d + 4 * q) = o[d];
+        if (q == 0) {
+            p.partial_ml[slot * 2] = m_run;
+            p.partial_ml[slot * 2 + 1] = l_run;
         }
     }
 }
@@ -210,7 +335,8 @@ __global__ __launch_bounds__(kThreads) void attention_kernel(const dlk_attention
 // loads are in flight together; dead splits are dropped by selection, never by a branch around the loads.
 constexpr int kCombineThreads = 512;
 
-template <int HD>
+// BASE2: attention_rows' partials, whose maxima are in base 2.
+template <int HD, bool BASE2>
 __global__ __launch_bounds__(kCombineThreads) void attention_combine(const dlk_attention_params p) {
     constexpr int GROUPS = kCombineThreads / HD;
     constexpr int WAVES = kCombineThreads / kWave;
@@ -243,10 +369,14 @@ __global__ __launch_bounds__(kCombineThreads) void attention_combine(const dlk_a
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            // a split without keys has weight 0 and an unwritten partial_o row: it must not enter the sum (0 * a
-            // stale NaN or Inf would), so it is selected away
-            const bool live = s0 + u * GROUPS < p.splits && ls[u] > 0.0f && ms[u] != -INFINITY;
-            const float w = live ? expf(ms[u] - maximum) : 0.0f;
+            // a split without keys has weight 0.  attention_rows writes its partials all the same (BASE2), and what its
+            // zero probabilities made of an infinity or NaN of V stays in the sum; the other kernels leave the row
+            // unwritten, so it is selected away (0 * a stale NaN or Inf must not enter)
+            const bool in = s0 + u * GROUPS < p.splits;
+            const bool live = BASE2 ? in : in && ls[u] > 0.0f && ms[u] != -INFINITY;
+            const float w = !live   ? 0.0f
+                            : BASE2 ? __builtin_amdgcn_exp2f(ms[u] - (maximum == -INFINITY ? 0.0f : maximum))
+                                    : expf(ms[u] - maximum);
             total += live ? w * ls[u] : 0.0f;
             acc += live ? w * o[u] : 0.0f;
         }
@@ -339,30 +469,30 @@ int launch_small(const dlk_attention_params& p, hipStream_t stream) {
                        p);
     int status = static_cast<int>(hipGetLastError());
     if (status != 0 || p.splits == 1 || p.partials_only) return status;
-    hipLaunchKernelGGL((attention_combine<HD>), dim3(static_cast<unsigned>(rows)), dim3(kCombineThreads), 0, stream, p);
+    hipLaunchKernelGGL((attention_combine<HD, false>), dim3(static_cast<unsigned>(rows)), dim3(kCombineThreads), 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
-template <int HD>
+template <int HD, bool BASE2 = false>
 int launch_combine(const dlk_attention_params& p, hipStream_t stream) {
     const int64_t combine_rows = static_cast<int64_t>(p.B) * p.H * p.L;
-    hipLaunchKernelGGL((attention_combine<HD>), dim3(static_cast<unsigned>(combine_rows)), dim3(kCombineThreads), 0, stream, p);
+    hipLaunchKernelGGL((attention_combine<HD, BASE2>), dim3(static_cast<unsigned>(combine_rows)), dim3(kCombineThreads), 0, stream, p);
     return static_cast<int>(hipGetLastError());
 }
 
+// The fewest row tiles per work-group that hold the rows of a KV head: the waves left over share the keys.
 template <typename KT, int HD>
 int launch(const dlk_attention_params& p, hipStream_t stream) {
-    // 64-key tiles; f32 K/V with 128-wide heads use 32-key tiles to keep the LDS footprint under 64 KB
-    constexpr int T = sizeof(KT) * HD > 256 ? 32 : 64;
-    const int G = p.H / p.KV;
-    const int row_blocks = (G * p.L + kRowsMax - 1) / kRowsMax;
-    dim3 grid(p.splits, row_blocks, p.B * p.KV);
-    hipLaunchKernelGGL((attention_kernel<KT, HD, T>), grid, dim3(kThreads), 0, stream, p);
-    int status = static_cast<int>(hipGetLastError());
+    const int rows = p.H / p.KV * p.L;
+    const int wr = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+    const dim3 grid(p.splits, (rows + 16 * wr - 1) / (16 * wr), p.B * p.KV);
+    const dim3 threads(kThreads);
+    if (wr == 1) hipLaunchKernelGGL((attention_rows<KT, HD, 1>), grid, threads, 0, stream, p);
+    else if (wr == 2) hipLaunchKernelGGL((attention_rows<KT, HD, 2>), grid, threads, 0, stream, p);
+    else hipLaunchKernelGGL((attention_rows<KT, HD, 4>), grid, threads, 0, stream, p);
+    const int status = static_cast<int>(hipGetLastError());
     if (status != 0 || p.splits == 1 || p.partials_only) return status;
-    const int64_t combine_rows = static_cast<int64_t>(p.B) * p.H * p.L;
-    hipLaunchKernelGGL((attention_combine<HD>), dim3(static_cast<unsigned>(combine_rows)), dim3(kCombineThreads), 0, stream, p);
-    return static_cast<int>(hipGetLastError());
+    return launch_combine<HD, true>(p, stream);
 }
 
 } // namespace
@@ -399,12 +529,17 @@ extern "C" int dlk_attention_scratch(int device, float** address) {
     return 0;
 }
 
+extern "C" int dlk_attention_takes_strides(const dlk_attention_params* p) {
+    return p->hd >= 16 && !dlk_attention_matrix_eligible(p) && !dlk_attention_prefill_eligible(p);
+}
+
 extern "C" int dlk_attention(const dlk_attention_params* params, dlh_stream stream_handle) {
     hipStream_t stream = reinterpret_cast<hipStream_t>(stream_handle);
     const dlk_attention_params& p = *params;
     if (p.B <= 0 || p.L <= 0 || p.KV <= 0 || p.H % p.KV != 0 || p.splits <= 0 || p.chunk <= 0 ||
         (p.splits > 1 && (!p.partial_o || !p.partial_ml)) || (p.splits > 1 && p.chunk % 64 != 0))
         return static_cast<int>(hipErrorInvalidValue);
+    if (p.q_row && !dlk_attention_takes_strides(&p)) return static_cast<int>(hipErrorInvalidValue);
     // a keep mask is applied by the general and small-head kernels, which serve non-causal attention
     if (p.keep_mask && (p.causal || p.qkv_partial || p.stage_out || p.kv_split)) return static_cast<int>(hipErrorInvalidValue);
     // the QKV projection's partials are finished only by the matrix kernel

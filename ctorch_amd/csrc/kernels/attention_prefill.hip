@@ -524,10 +524,13 @@ __global__ __launch_bounds__(kThreads, sizeof(KT) == 2 ? 2 : 1) void attention_p
 } // namespace dlk
 
 /* Whether dlk_attention takes the matrix-core prefill kernel for these parameters. */
+extern "C" int dlk_attention_prefill_heads(int heads, int kv_heads, int head_dim, int length) {
+    const int G = kv_heads > 0 ? heads / kv_heads : 0;
+    return (head_dim == 64 || head_dim == 128) && length >= 16 && G > 0 && dlk::kRows % G == 0;
+}
+
 extern "C" int dlk_attention_prefill_eligible(const dlk_attention_params* p) {
-    const int G = p->KV > 0 ? p->H / p->KV : 0;
-    return p->causal && !p->keep_mask && (p->hd == 64 || p->hd == 128) && p->L >= 16 && G > 0 && dlk::kRows % G == 0 &&
-           p->splits == 1 && p->ldq % 4 == 0 && p->ldo % 4 == 0;
+    return p->causal && !p->keep_mask && dlk_attention_prefill_heads(p->H, p->KV, p->hd, p->L) && p->splits == 1 && p->ldq % 4 == 0 && p->ldo % 4 == 0;
 }
 
 extern "C" int64_t dlk_attention_split_bytes(const dlk_attention_params* p) {

@@ -187,6 +187,9 @@ typedef struct dlk_attention_params {
        of keys starts below it requests its first K/V tile before it reads the device length.  A hint for speed
        only: any value gives the same result. */
     int64_t early_keys;
+    /* General kernel (head dim 16 and up): element strides of the query per sequence, position and head where its rows
+       are not [B * L, ldq]; q_row 0: they are. */
+    int64_t q_batch, q_row, q_head;
 } dlk_attention_params;
 
 /* Keys per split of a short one-position decode over a bf16 cache (few keys in all): 256 or 512, one work-group. */
@@ -199,6 +202,8 @@ int dlk_attention_matrix_heads(int heads, int kv_heads, int head_dim);
 
 
 int dlk_attention(const dlk_attention_params* p, dlh_stream stream);
+/* 1 when dlk_attention takes the general kernel for these parameters, which reads the query through its strides. */
+int dlk_attention_takes_strides(const dlk_attention_params* p);
 /* Floats of the device-resident scratch array behind the allocation-free attention entry (8 MiB per GPU). */
 #define DLK_ATTENTION_SCRATCH_FLOATS (2 << 20)
 /* The address of that array on GPU `device` (looked up once per device with the device current; later calls
@@ -207,6 +212,8 @@ int dlk_attention_scratch(int device, float** address);
 /* The matrix-core causal prefill kernel (attention_prefill.hip), which dlk_attention takes for causal launches
    over bf16 or f32 K/V, head dim 64 or 128, L >= 16 new positions, one split and H/KV dividing 128. */
 int dlk_attention_prefill_eligible(const dlk_attention_params* p);
+/* Its part about the heads and the chunk: head dim 64 or 128, L >= 16, H/KV dividing 128. */
+int dlk_attention_prefill_heads(int heads, int kv_heads, int head_dim, int length);
 /* One position on the matrix cores (attention_matrix.hip): eligibility, and the launch of the attention kernel
    alone (with several splits it writes the partials; dlk_attention adds the merge). */
 int dlk_attention_matrix_eligible(const dlk_attention_params* p);

@@ -265,7 +265,7 @@ Tensor GroupedQueryAttention::run(const Tensor& input, KVCache* cache) {
     a.causal = 1;
     a.out = static_cast<float*>(mutable_data(attended));
     a.ldo = d;
-    attention_split(B, heads_, kv_heads_, hd, a.kv_bf16 != 0, L, offset + L, a.splits, a.chunk);
+    attention_split(B, heads_, kv_heads_, hd, a.kv_bf16 != 0, L, offset + L, true, a.splits, a.chunk);
     Tensor po, pml;
     if (a.splits > 1) {
         po = empty_tensor({B * heads_ * L, a.splits, hd}, DType::f32, input.device());
@@ -320,7 +320,7 @@ Tensor TransformerDecoderLayer::decode(const Tensor& input, KVCache& cache) {
     DecodeWorkspace ws;
     int splits = 1, chunk = 64;
     attention_split(B, attention_->heads(), attention_->kv_heads(), attention_->head_dim(),
-                    cache_dtype(*this) == DType::bf16, L, cache.length() + L, splits, chunk);
+                    cache_dtype(*this) == DType::bf16, L, cache.length() + L, true, splits, chunk);
     decode_layer(*this, x.data<float>(), static_cast<float*>(mutable_data(out)), B, L, cache, ws, splits, chunk, context);
     return out;
 }
@@ -387,7 +387,7 @@ Tensor TransformerDecoder::decode(const Tensor& input, std::span<KVCache> cache)
         int splits = 1, chunk = 64;
         const auto& front = layers_.front()->attention();
         attention_split(B, front.heads(), front.kv_heads(), front.head_dim(),
-                        detail::cache_dtype(*layers_.front()) == DType::bf16, L, prefix + L, splits, chunk);
+                        detail::cache_dtype(*layers_.front()) == DType::bf16, L, prefix + L, true, splits, chunk);
         for (std::size_t i = 0; i < layers_.size(); ++i) {
             cache[i].reserve(B, layers_[i]->attention().kv_heads(), layers_[i]->attention().head_dim(),
                              detail::cache_dtype(*layers_[i]), input.device());

@@ -80,7 +80,7 @@ void linear_into(const float* x, Index rows, Index k, const Tensor& weight, cons
 }
 
 void attention_split(Index batch, Index heads, Index kv_heads, Index head_dim, bool kv_bf16, Index length,
-                     Index source, int& splits, int& chunk) {
+                     Index source, bool causal, int& splits, int& chunk) {
     constexpr Index tile = 64;
     const bool matrix = dlk_attention_matrix_heads(static_cast<int>(heads), static_cast<int>(kv_heads),
                                                    static_cast<int>(head_dim)) != 0;
@@ -115,13 +115,20 @@ void attention_split(Index batch, Index heads, Index kv_heads, Index head_dim, b
         splits = static_cast<int>(std::max<Index>(1, (source + per - 1) / per));
         return;
     }
-    const Index groups = batch * kv_heads;
+    // several positions.  A causal chunk that the prefill kernel takes spreads over its query rows and is never split
+    splits = 1;
+    chunk = static_cast<int>((source + tile - 1) / tile * tile);
+    if (causal && dlk_attention_prefill_heads(static_cast<int>(heads), static_cast<int>(kv_heads),
+                                              static_cast<int>(head_dim), static_cast<int>(length)))
+        return;
+    // the others (attention_rows, a work-group per 64 rows of a KV head): key splits of two or more 64-key tiles until
+    // every CU has a work-group.  Measured on MI355X at 4 sequences x 7 positions over 1508 keys (32 such groups), us a
+    // layer with its merge: 8 splits 16.3, 12 17.2, 24 (one tile each) 17.4; with 256 groups already (4 x 510 byte
+    // positions) 3 splits took 58 against 19.
+    const Index groups = (heads / kv_heads * length + 63) / 64 * batch * kv_heads;
+    const Index wanted = std::max<Index>(1, 256 / groups);
     const Index tiles = std::max<Index>(1, (source + tile - 1) / tile);
-    Index wanted = 1;
-    // decode: enough key splits for ~2 work-groups per CU slot of a 256-CU chip; prefill rows already spread
-    if (length <= 4) wanted = std::max<Index>(1, (1024 + groups - 1) / groups);
-    wanted = std::min(wanted, tiles);
-    const Index per = (tiles + wanted - 1) / wanted;
+    const Index per = std::max<Index>(2, (tiles + wanted - 1) / wanted);
     splits = static_cast<int>((tiles + per - 1) / per);
     chunk = static_cast<int>(per * tile);
 }
@@ -219,13 +226,11 @@ Tensor grouped_query_attention(const Tensor& query, const Tensor& key, const Ten
         throw std::invalid_argument("grouped_query_attention: shapes differ or H is not a multiple of KV");
     if (D != 2 && D != 4 && D != 8 && D != 16 && D != 32 && D != 64 && D != 128)
         throw std::invalid_argument("grouped_query_attention: head size 2, 4, 8, 16, 32, 64 or 128");
-    Tensor q = contiguous_f32(query.transpose(1, 2)); // [B, L, H, D] = rows (b, l)
     const DType kv_dtype = key.dtype() == DType::bf16 && value.dtype() == DType::bf16 ? DType::bf16 : DType::f32;
     Tensor k = key.dtype() == kv_dtype && key.is_contiguous() ? key : key.astype(kv_dtype).contiguous();
     Tensor v = value.dtype() == kv_dtype && value.is_contiguous() ? value : value.astype(kv_dtype).contiguous();
     Tensor out = empty_tensor({B, L, H, D}, DType::f32, query.device());
     dlk_attention_params p{};
-    p.q = q.data<float>();
     p.ldq = H * D;
     p.k = k.data<void>();
     p.v = v.data<void>();
@@ -264,7 +269,7 @@ Tensor grouped_query_attention(const Tensor& query, const Tensor& key, const Ten
         }
         p.keep_mask = static_cast<const unsigned char*>(mask.data<void>());
     }
-    attention_split(B, H, KV, D, kv_dtype == DType::bf16, L, S, p.splits, p.chunk);
+    attention_split(B, H, KV, D, kv_dtype == DType::bf16, L, S, false, p.splits, p.chunk);
     Tensor po, pml;
     if (p.splits > 1) {
         po = empty_tensor({B * H * L, p.splits, D}, DType::f32, query.device());
@@ -272,6 +277,16 @@ Tensor grouped_query_attention(const Tensor& query, const Tensor& key, const Ten
         p.partial_o = static_cast<float*>(mutable_data(po));
         p.partial_ml = static_cast<float*>(mutable_data(pml));
     }
+    // the general kernel reads an f32 query where it lies, the others rows (b, l) of [B, L, H, D]
+    Tensor q = query;
+    if (query.dtype() == DType::f32 && query.strides()[3] == 1 && query.strides()[2] > 0 && dlk_attention_takes_strides(&p)) {
+        p.q_batch = query.strides()[0];
+        p.q_head = query.strides()[1];
+        p.q_row = query.strides()[2];
+    } else {
+        q = contiguous_f32(query.transpose(1, 2));
+    }
+    p.q = q.data<float>();
     hip_check(dlk_attention(&p, context.stream), "grouped_query_attention");
     return out.transpose(1, 2);
 }

@@ -22,6 +22,6 @@ void linear_into(const float* x, Index rows, Index k, const Tensor& weight, cons
 
 /// Number of key splits and keys per split for attention of `length` new positions over `source` keys.
 void attention_split(Index batch, Index heads, Index kv_heads, Index head_dim, bool kv_bf16, Index length,
-                     Index source, int& splits, int& chunk);
+                     Index source, bool causal, int& splits, int& chunk);
 
 } // namespace dl::detail

@@ -1,0 +1,90 @@
+"""The general attention kernel (several positions, masks, head sizes 16 to 128) against numpy in 64 bits: edges of its
+row tiles and key tiles, key splits, queries read through strides, and the causal chunks of a decoder against the oracle."""
+import numpy as np
+import pytest
+
+import ctorch_amd as ct
+import oracle
+from common import build_pair, rel_err, say
+
+pytestmark = pytest.mark.gpu
+GPU = ct.device("gpu")
+
+
+def reference(q, k, v, mask):
+    group = q.shape[1] // k.shape[1]
+    q, k, v = q.astype(np.float64), np.repeat(k, group, 1).astype(np.float64), np.repeat(v, group, 1).astype(np.float64)
+    s = q @ k.transpose(0, 1, 3, 2) / np.sqrt(q.shape[-1])
+    if mask is not None:
+        s = np.where(mask, s, -np.inf)
+    with np.errstate(invalid="ignore"):
+        e = np.exp(s - s.max(-1, keepdims=True))
+        return (e / e.sum(-1, keepdims=True)) @ v
+
+
+@pytest.mark.parametrize("B,H,KV,L,S,D,bf16,masked", [
+    (1, 2, 2, 1, 1, 16, False, False), (2, 3, 1, 5, 65, 32, False, True), (1, 8, 2, 4, 128, 64, True, False),
+    (2, 12, 4, 11, 129, 64, False, True), (1, 4, 4, 65, 300, 128, True, True), (4, 32, 8, 7, 1508, 64, False, False),
+    (1, 16, 2, 9, 700, 128, False, False), (1, 40, 2, 1, 200, 64, False, False), (2, 6, 2, 50, 50, 16, True, True)])
+def test_attention_rows_match_64_bit_results(B, H, KV, L, S, D, bf16, masked):
+    say(f"case: attention B={B} H={H} KV={KV} L={L} S={S} D={D} bf16={bf16} masked={masked}")
+    rng = np.random.default_rng(S + L)
+    q = rng.standard_normal((B, H, L, D)).astype(np.float32)
+    k, v = (rng.standard_normal((B, KV, S, D)).astype(np.float32) for _ in range(2))
+    if bf16:
+        kb, vb = oracle.bf16_encode(k), oracle.bf16_encode(v)
+        k, v = oracle.bf16_decode(kb), oracle.bf16_decode(vb)
+        gk, gv = (ct.Tensor.from_numpy(a, ct.BF16, GPU) for a in (kb, vb))
+    else:
+        gk, gv = (ct.Tensor.from_numpy(a, ct.F32, GPU) for a in (k, v))
+    masks = [None]
+    if masked:
+        shared = rng.random((B, 1, 1, S)) < 0.6
+        shared[:, :, :, S // 2:] = False      # whole tiles dropped
+        shared[:, :, :, 0] = True
+        own = rng.random((1, H, L, S)) < 0.5
+        own[0, 0, 0] = False                  # a row that keeps no key
+        masks = [shared, own]
+    want_nan = [m is not None and m.shape[1] > 1 for m in masks]
+    for mask, nan in zip(masks, want_nan):
+        gm = None if mask is None else ct.Tensor.from_numpy(mask, ct.BOOL, GPU)
+        want = reference(q, k, v, mask)
+        assert np.isnan(want).any() == nan
+        # the query as stored, and as a [B, L, H, D] tensor's transposed view would be made contiguous by the caller
+        got = ct.grouped_query_attention(ct.Tensor.from_numpy(q, ct.F32, GPU), gk, gv, gm).numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        # f32 sums: a score is off by some |score| 2^-24 sqrt(D), a weighted sum by 2^-24 sqrt(S)
+        error = np.nan_to_num(got - want)
+        assert np.linalg.norm(error) <= 2.0**-24 * (np.sqrt(D) + np.sqrt(S) + 8) * np.linalg.norm(np.nan_to_num(want))
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_a_nan_value_under_the_mask_reaches_every_row_as_in_the_reference(bf16):
+    say("case: attention, a NaN in V only under a mask that drops whole tiles")
+    rng = np.random.default_rng(5)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((1, 4, 3, 64), (1, 2, 256, 64), (1, 2, 256, 64)))
+    mask = np.ones((1, 1, 1, 256), bool)
+    mask[..., 128:] = False
+    v[:, 0, 200, 3] = np.nan  # zero times NaN: head-dim entry 3 of the two query heads of KV head 0
+    bits = (lambda a: ct.Tensor.from_numpy(oracle.bf16_encode(a), ct.BF16, GPU)) if bf16 else (
+        lambda a: ct.Tensor.from_numpy(a, ct.F32, GPU))
+    got = ct.grouped_query_attention(ct.Tensor.from_numpy(q, ct.F32, GPU), bits(k), bits(v),
+                                     ct.Tensor.from_numpy(mask, ct.BOOL, GPU)).numpy()
+    want = np.zeros(got.shape, bool)
+    want[:, :2, :, 3] = True
+    assert np.array_equal(np.isnan(got), want)
+
+
+@pytest.mark.parametrize("batch,prefix,length,heads,kv,hd,kv_dtype", [
+    (2, 100, 7, 8, 2, 64, None), (1, 700, 15, 8, 4, 128, None), (2, 63, 2, 8, 8, 64, ct.BF16), (3, 200, 33, 8, 2, 32, None),
+    (1, 130, 20, 6, 2, 64, None)])
+def test_causal_chunks_over_a_prefix_match_the_oracle(batch, prefix, length, heads, kv, hd, kv_dtype):
+    say(f"case: {length} new positions over {prefix}, heads {heads}/{kv} of {hd}")
+    cfg = oracle.ModelConfig(vocab=64, layers=2, dimensions=heads * hd, heads=heads, kv_heads=kv, hidden=256,
+                             context=prefix + length + 2, dtype="f32")
+    ref, gpu = build_pair(cfg, root=(91, 0), kv_dtype=kv_dtype)
+    ids = oracle.random_ids((92, 0), batch * (prefix + length), cfg.vocab).reshape(batch, -1)
+    rc, gc = ref.make_cache(batch), gpu.cache()
+    bound = 1e-4 if kv_dtype is None else 2e-2
+    for part in (ids[:, :prefix], ids[:, prefix:]):
+        assert rel_err(gpu.logits(part, gc), ref.logits(part, rc)[:, -1]) <= bound
