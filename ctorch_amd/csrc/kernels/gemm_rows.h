@@ -142,6 +142,8 @@ __device__ __forceinline__ const uint16_t* tile_row(const TileMap& t, int i, int
 }
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef short s16x4 __attribute__((ext_vector_type(4))); // the bf16 operands of v_mfma_f32_16x16x16_bf16
@@ -221,8 +223,19 @@ __device__ __forceinline__ void lane_epilogue(const dlk_gemv_params& p, const Ti
                                               RowPosition where = {0, 0, false}) {
     if constexpr (EPI == DLK_EPI_SWIGLU) {
         const int n = t.n0 + 2 * q;
-        p.y[static_cast<int64_t>(m) * p.ldy + n] = gemv::silu(v[0]) * v[1];
-        p.y[static_cast<int64_t>(m) * p.ldy + n + 1] = gemv::silu(v[2]) * v[3];
+        const float o0 = gemv::silu(v[0]) * v[1], o1 = gemv::silu(v[2]) * v[3];
+        if (p.stage_out) {
+            // the reduce of a staged launch: the pair's bf16 hi and lo in the next launch's staging layout (gemm_tiles.h)
+            char* at = static_cast<char*>(p.stage_out) + (static_cast<int64_t>(m / 16) * (p.seg_rows[0] / 32) + n / 32) * 2048 +
+                       ((m % 16) + 16 * ((n % 32) / 8)) * 16 + (n % 8) * 2;
+            const f32x2 o = {o0, o1};
+            const bf16x2 h = __builtin_convertvector(o, bf16x2);
+            *reinterpret_cast<bf16x2*>(at) = h;
+            *reinterpret_cast<bf16x2*>(at + 1024) = __builtin_convertvector(o - __builtin_convertvector(h, f32x2), bf16x2);
+            return;
+        }
+        p.y[static_cast<int64_t>(m) * p.ldy + n] = o0;
+        p.y[static_cast<int64_t>(m) * p.ldy + n + 1] = o1;
     } else if constexpr (EPI == DLK_EPI_STORE || EPI == DLK_EPI_RESIDUAL) {
         // every operand is loaded before the first store: y may alias them as far as the compiler knows, so a
         // load issued after a store waits for it, and the four outputs would take four memory round trips

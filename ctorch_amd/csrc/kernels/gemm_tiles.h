@@ -38,7 +38,6 @@ using gemv::u32x4;
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 constexpr int kThreads = 512;                      // 8 waves
 constexpr int kWaves = kThreads / kWave;
-constexpr int kPrepThreads = 256;                  // prepare_rows: one work-group per 16-row tile and k chunk
 constexpr int kPrepChunk = 512;                    // k per prepare_rows work-group
 constexpr int kBN = 256;                           // weight rows per work-group (16 tiles of 16)
 constexpr int kBM = 256;                           // activation rows per work-group (16 tiles of 16)
@@ -105,12 +104,6 @@ inline bool shape_eligible(const dlk_gemv_params& p) {
     return row_blocks(p) >= 2 || col_blocks(p) >= kMinBlocks;
 }
 
-/// The tiled path runs when the shape suits it and the caller attached the staging workspace.
-inline bool eligible(const dlk_gemv_params& p) {
-    return shape_eligible(p) && p.stage && p.stage_bytes >= stage_bytes(p) &&
-           reinterpret_cast<uintptr_t>(p.stage) % 16 == 0;
-}
-
 // Work-group barrier for the DMA ring: the caller has waited for its own DMA; no fence (a fence over LDS would
 // wait for every DMA in flight).  The empty asm keeps the compiler from moving LDS accesses across it.
 __device__ __forceinline__ void ring_barrier() {
@@ -134,12 +127,11 @@ __device__ __forceinline__ const char* tile_base(const dlk_gemv_params& p, int n
 }
 
 // Preparation launch: work-group (mt, c) splits rows 16 mt .. +16 over k chunk c (512 wide).  Wave w takes the
-// chunk's k steps w, w + 4, ...; lane l (row 16 mt + l % 16, k 32 s + 8 (l / 16) .. +8) writes hi + lo = x * g
+// chunk's k steps w, w + waves, ...; lane l (row 16 mt + l % 16, k 32 s + 8 (l / 16) .. +8) writes hi + lo = x * g
 // (bf16 pair, the remainder rounded once more) at 16 l of the step's two 1 KB blocks, so every wave writes whole
 // 1 KB blocks.  With the norm the work-group writes the chunk's sum of squares of x (f32) for each row.
-template <bool NORM>
-__global__ __launch_bounds__(kPrepThreads) void prepare_rows(const dlk_gemv_params p) {
-    constexpr int kPrepWaves = kPrepThreads / kWave;
+template <bool NORM, int kPrepWaves>
+__global__ __launch_bounds__(kPrepWaves * kWave) void prepare_rows(const dlk_gemv_params p) {
     __shared__ float partial[kPrepWaves][16];
     const int t = threadIdx.x, lane = t % kWave, wave = t / kWave, K = p.K, nsteps = K / 32;
     const int mt = blockIdx.x, chunk = blockIdx.y, r = lane % 16, q = lane / 16;
@@ -576,9 +568,12 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_tiles(const dlk_gemv_params 
 constexpr int kNarrowWaves = 4; // waves (16-row tiles) per work-group
 constexpr int kNarrowBatch = 4; // k steps per batch of loads (two batches in flight)
 
-/// Whether a tiled-eligible launch takes gemm_narrow (host side).
+/// Whether a staged launch takes gemm_narrow (host side).
 inline bool narrow_eligible(const dlk_gemv_params& p) {
-    return p.epilogue == DLK_EPI_STORE && !p.bias && gemm::tiles_of(p) <= 2;
+    for (int s = 0; s < p.nseg; ++s)
+        if (p.seg_rows[s] % gemm::kTile != 0) return false;
+    return p.epilogue == DLK_EPI_STORE && !p.bias && gemm::tiles_of(p) <= 2 && p.ldy % 4 == 0 &&
+           reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
 }
 
 template <bool NORM>

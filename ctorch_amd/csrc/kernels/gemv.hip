@@ -1,13 +1,13 @@
 // Host dispatch of the projections: the GEMV (gemv_impl.h) for one or two activation rows (or shapes the matrix
 // cores do not take), the matrix-core kernel (gemm_rows.h) for a batch of decode rows, and the tiled matrix-core
-// kernel (gemm_tiles.h) for prefill chunks large enough to fill the device, and with f32 weights the f32 matrix-core
-// kernel (gemm_f32.h); all instantiated per epilogue in gemv_*.hip.
+// kernels for prompts and prefill chunks (gemm_tiles.h, gemm_mid.h where its tiles would not fill the device), and with
+// f32 weights the f32 matrix-core kernel (gemm_f32.h); all instantiated per epilogue in gemv_*.hip.
 //
 // The grid is persistent: one wave per row group, capped at the number of waves the chosen kernel keeps
 // resident on the device (its occupancy times the CU count), so every wave streams from the start and none
 // waits for another to retire.  LOGITS launches write one sampling candidate per work-group.
 #include "kernels/gemm_f32.h"
-#include "kernels/gemm_tiles.h"
+#include "kernels/gemm_mid.h"
 
 #include <mutex>
 #include <unordered_map>
@@ -61,7 +61,65 @@ Kernel resolve_tiles(const dlk_gemv_params& p) {
     }
 }
 
+/// A shape that one of the staged kernels (gemm_tiles, gemm_mid, gemm_narrow) takes.
+bool staged_shape(const dlk_gemv_params& p) { return dlk::tiles::shape_eligible(p) || dlk::mid::shape_eligible(p); }
+
+/// The staged kernels run when the shape suits one and the caller attached the staging workspace.
+bool staged(const dlk_gemv_params& p) {
+    return p.stage && reinterpret_cast<uintptr_t>(p.stage) % 16 == 0 && staged_shape(p) &&
+           p.stage_bytes >= dlk::tiles::stage_bytes(p);
+}
+
+// Which of the two kernels a staged launch takes where both fit: the one whose work-groups, one per CU at a time, need
+// less time.  Measured on MI355X at K = 4096 a round of 128 x 128 tiles takes 63 us and one of 256 x 256 tiles 181 us:
+// 1013 rows -> 6144 (384 or 96 work-groups) 114 against 157 us, 333 rows 2048 -> 32000 (750 or 250) 99 and 95, 2000 rows
+// -> 16000 (2000 or 504) 271 against 199.
+bool use_mid(const dlk_gemv_params& p) {
+    if (!dlk::mid::shape_eligible(p)) return false;
+    if (!dlk::tiles::shape_eligible(p)) return true;
+    auto rounds = [](int64_t blocks) { return (blocks + 255) / 256; };
+    return rounds(static_cast<int64_t>(dlk::mid::col_blocks(p)) * dlk::mid::row_blocks(p)) * 63 <
+           rounds(static_cast<int64_t>(dlk::tiles::col_blocks(p)) * dlk::tiles::row_blocks(p)) * 181;
+}
+
+Kernel resolve_reduce(const dlk_gemv_params& p);
+
+int launch_reduce(dlk_gemv_params& p, int splits, hipStream_t stream) {
+    using namespace dlk::gemm;
+    const Kernel reduce = resolve_reduce(p);
+    if (!reduce.fn) return static_cast<int>(hipErrorInvalidValue);
+    const int64_t threads = static_cast<int64_t>(p.M) * tiles_of(p) * 4;
+    void* args[] = {&p, &splits};
+    return static_cast<int>(hipLaunchKernel(reduce.fn,
+                                            dim3(static_cast<unsigned>((threads + kReduceThreads - 1) / kReduceThreads)),
+                                            dim3(kReduceThreads), args, 0, stream));
+}
+
 int launch_prepare(const dlk_gemv_params& p, hipStream_t stream);
+
+// The staged rows through gemm_mid, and the sum of its key slices.
+int launch_mid(const dlk_gemv_params& params, hipStream_t stream) {
+    using namespace dlk::mid;
+    dlk_gemv_params p = params;
+    const void* kernel = nullptr;
+    switch (p.epilogue) {
+    case DLK_EPI_STORE: kernel = dlk_mid_kernel_store(p); break;
+    case DLK_EPI_RESIDUAL: kernel = dlk_mid_kernel_residual(p); break;
+    case DLK_EPI_QKV: kernel = dlk_mid_kernel_qkv(p); break;
+    case DLK_EPI_SWIGLU: kernel = dlk_mid_kernel_swiglu(p); break;
+    default: break;
+    }
+    if (!kernel) return static_cast<int>(hipErrorInvalidValue);
+    int splits = splits_of(p);
+    if (splits > 1 && (!p.split_partial || p.split_capacity < split_floats(p))) splits = 1;
+    if (splits > 1) p.bump_position = nullptr; // the reduce launch advances the length
+    void* args[] = {&p};
+    const int status = static_cast<int>(
+        hipLaunchKernel(kernel, dim3(col_blocks(p) * row_blocks(p), splits), dim3(kThreads), args, 0, stream));
+    if (status != 0 || splits == 1) return status;
+    p.bump_position = params.bump_position;
+    return launch_reduce(p, splits, stream);
+}
 
 // Tiled path: prepare_rows splits the activation rows into the staging workspace (unless the caller says it
 // already holds them), then the tiled projection.
@@ -73,6 +131,7 @@ int launch_tiles(const dlk_gemv_params& p, hipStream_t stream) {
     const int status = launch_prepare(p, stream);
     if (status != 0) return status;
     void* args[] = {const_cast<dlk_gemv_params*>(&p)};
+    if (!narrow.fn && use_mid(p)) return launch_mid(p, stream);
     if (narrow.fn) {
         const int waves = (p.M + 15) / 16;
         return static_cast<int>(hipLaunchKernel(kernel.fn, dim3((waves + kNarrowWaves - 1) / kNarrowWaves),
@@ -87,10 +146,15 @@ int launch_prepare(const dlk_gemv_params& p, hipStream_t stream) {
     if (p.stage_ready) return 0;
     void* args[] = {const_cast<dlk_gemv_params*>(&p)};
     const bool norm = p.apply_norm && p.epilogue != DLK_EPI_RESIDUAL;
-    const void* prep = norm ? reinterpret_cast<const void*>(&prepare_rows<true>)
-                            : reinterpret_cast<const void*>(&prepare_rows<false>);
-    return static_cast<int>(
-        hipLaunchKernel(prep, dim3((p.M + 15) / 16, prep_chunks(p.K)), dim3(kPrepThreads), args, 0, stream));
+    const dim3 grid((p.M + 15) / 16, prep_chunks(p.K));
+    // few work-groups: sixteen waves each, so that every load of a work-group is in flight at once (200 rows of 2048 5.8 ->
+    // 4.6 us; at 16384 rows four waves leave room for more work-groups per CU)
+    const bool few = static_cast<int64_t>(grid.x) * grid.y <= 1024;
+    const void* prep = norm ? (few ? reinterpret_cast<const void*>(&prepare_rows<true, 16>)
+                                   : reinterpret_cast<const void*>(&prepare_rows<true, 4>))
+                            : (few ? reinterpret_cast<const void*>(&prepare_rows<false, 16>)
+                                   : reinterpret_cast<const void*>(&prepare_rows<false, 4>));
+    return static_cast<int>(hipLaunchKernel(prep, grid, dim3((few ? 16 : 4) * dlk::kWave), args, 0, stream));
 }
 
 int launch_gemm(const dlk_gemv_params& params, hipStream_t stream) {
@@ -158,14 +222,8 @@ int launch_gemm(const dlk_gemv_params& params, hipStream_t stream) {
         if (p.defer_reduce) continue; // the attention finishes the projection
         if (splits > 1) {
             p.bump_position = const_cast<int64_t*>(bump);
-            const Kernel reduce = resolve_reduce(p);
-            if (!reduce.fn) return static_cast<int>(hipErrorInvalidValue);
-            const int64_t threads = static_cast<int64_t>(p.M) * tiles_of(p) * 4;
-            void* rargs[] = {&p, &splits};
-            status = hipLaunchKernel(reduce.fn,
-                                     dim3(static_cast<unsigned>((threads + kReduceThreads - 1) / kReduceThreads)),
-                                     dim3(kReduceThreads), rargs, 0, stream);
-            if (status != hipSuccess) return static_cast<int>(status);
+            const int reduced = launch_reduce(p, splits, stream);
+            if (reduced != 0) return reduced;
         }
     }
     return 0;
@@ -269,15 +327,15 @@ extern "C" int dlk_pack_tiles(const void* w0, const void* w1, int swiglu, int64_
 
 extern "C" int dlk_gemv_uses_rows(const dlk_gemv_params* p) {
     // both matrix-core kernels of the batched path (gemm_rows, gemm_wide) read the repacked weights
-    return !dlk::tiles::eligible(*p) && dlk::gemm::eligible(*p) ? 1 : 0;
+    return !staged(*p) && dlk::gemm::eligible(*p) ? 1 : 0;
 }
 
 extern "C" int dlk_gemv_folds_lora(const dlk_gemv_params* p) {
-    return !dlk::tiles::eligible(*p) && dlk::gemm::eligible(*p) && dlk::gemm::lora_fold_eligible(*p) ? 1 : 0;
+    return !staged(*p) && dlk::gemm::eligible(*p) && dlk::gemm::lora_fold_eligible(*p) ? 1 : 0;
 }
 
 extern "C" int64_t dlk_gemv_split_floats(const dlk_gemv_params* p) {
-    if (dlk::tiles::eligible(*p)) return 0;
+    if (staged(*p)) return !dlk_tiles_kernel_narrow(*p).fn && use_mid(*p) ? dlk::mid::split_floats(*p) : 0;
     if (!dlk::gemm::eligible(*p)) return 0;
     const int rows = std::min(p->M, dlk::gemm::kMaxRows);
     return dlk::gemm::split_floats(*p, dlk::gemm::splits_of(*p, rows), rows);
@@ -285,7 +343,7 @@ extern "C" int64_t dlk_gemv_split_floats(const dlk_gemv_params* p) {
 
 extern "C" int dlk_gemv_split_count(const dlk_gemv_params* p) {
     using namespace dlk::gemm;
-    if (dlk::tiles::eligible(*p) || !eligible(*p) || p->M > kMaxRows || wide_eligible(*p) || wide_parts_eligible(*p))
+    if (staged(*p) || !eligible(*p) || p->M > kMaxRows || wide_eligible(*p) || wide_parts_eligible(*p))
         return 1;
     int splits = splits_of(*p, p->M);
     if (splits > 1 && (!p->split_partial || p->split_capacity < split_floats(*p, splits, p->M))) splits = 1;
@@ -294,7 +352,7 @@ extern "C" int dlk_gemv_split_count(const dlk_gemv_params* p) {
 }
 
 extern "C" int64_t dlk_gemv_stage_bytes(const dlk_gemv_params* p) {
-    return dlk::tiles::shape_eligible(*p) ? dlk::tiles::stage_bytes(*p) : 0;
+    return staged_shape(*p) ? dlk::tiles::stage_bytes(*p) : 0;
 }
 
 extern "C" int dlk_gemv_blocks(const dlk_gemv_params* p) {
@@ -319,16 +377,16 @@ extern "C" int dlk_gemv(const dlk_gemv_params* params, dlh_stream stream_handle)
         for (int s = 0; s < params->nseg; ++s)
             if (params->seg_rows[s] % 2 != 0 || params->head_dim % 2 != 0) return static_cast<int>(hipErrorInvalidValue);
     // the staged SwiGLU output exists only on the tiled path
-    if (params->stage_out && (params->epilogue != DLK_EPI_SWIGLU || !dlk::tiles::eligible(*params) ||
+    if (params->stage_out && (params->epilogue != DLK_EPI_SWIGLU || !staged(*params) ||
                               params->seg_rows[0] % 32 != 0 || reinterpret_cast<uintptr_t>(params->stage_out) % 16 != 0))
         return static_cast<int>(hipErrorInvalidValue);
-    if (params->defer_reduce && (dlk::tiles::eligible(*params) || !dlk::gemm::eligible(*params) ||
+    if (params->defer_reduce && (staged(*params) || !dlk::gemm::eligible(*params) ||
                                  dlk::gemm::wide_eligible(*params)))
         return static_cast<int>(hipErrorInvalidValue);
     // only the wide kernel applies LoRA down rows
     if ((params->lora_down[0] || params->lora_down[1] || params->lora_down[2]) && !dlk_gemv_folds_lora(params))
         return static_cast<int>(hipErrorInvalidValue);
-    if (dlk::tiles::eligible(*params)) return launch_tiles(*params, stream);
+    if (staged(*params)) return launch_tiles(*params, stream);
     if (dlk::gemm::eligible(*params)) return launch_gemm(*params, stream);
     if (dlk::gemm32::eligible(*params)) return launch_f32(*params, stream);
     const int waves = launch_waves(*params);

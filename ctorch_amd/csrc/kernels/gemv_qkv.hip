@@ -1,6 +1,6 @@
 // Projection kernels with the QKV epilogue: the GEMV (one activation row) and the matrix-core variant.
 #include "kernels/gemm_f32.h"
-#include "kernels/gemm_tiles.h"
+#include "kernels/gemm_mid.h"
 
 dlk::gemv::Kernel dlk_gemv_kernel_qkv(const dlk_gemv_params& p, int mt) {
     return dlk::gemv::resolve<DLK_EPI_QKV>(p, mt);
@@ -20,4 +20,8 @@ dlk::gemv::Kernel dlk_tiles_kernel_qkv(const dlk_gemv_params& p) {
 
 const void* dlk_gemm_f32_kernel_qkv(const dlk_gemv_params& p, int shape) {
     return dlk::gemm32::resolve<DLK_EPI_QKV>(p, shape);
+}
+
+const void* dlk_mid_kernel_qkv(const dlk_gemv_params& p) {
+    return dlk::mid::resolve<DLK_EPI_QKV>(p);
 }

@@ -89,7 +89,7 @@ typedef struct dlk_gemv_params {
      * per-row sums of squares of each key slice, reduced in fixed order by a second launch. */
     float* split_partial;
     int64_t split_capacity; /* floats */
-    /* Workspace of the tiled (prefill) path: a preparation launch writes the activation rows (times the norm
+    /* Workspace of the staged (prompt and prefill) path: a preparation launch writes the activation rows (times the norm
      * weight) split into bf16 hi + lo rows and the per-row norm factors.  NULL: many-row launches take the
      * batched matrix-core path (64 rows per launch) instead. */
     void* stage;

@@ -43,6 +43,8 @@ Tensor SwiGLU::forward(const Tensor& input) {
     p.w_bf16 = gb;
     p.y = static_cast<float*>(mutable_data(act));
     p.ldy = F;
+    DecodeWorkspace ws;
+    ws.attach_workspace(p, input.device());
     hip_check(dlk_gemv(&p, context.stream), "SwiGLU gate/up");
     return linear(act, down_->weight(), down_->bias());
 }
@@ -248,6 +250,8 @@ Tensor GroupedQueryAttention::run(const Tensor& input, KVCache* cache) {
     adapter_hidden(query_adapter_.get(), lq, 0);
     adapter_hidden(value_adapter_.get(), lv, 2);
     if (d % (qb ? 8 : 4) != 0) throw std::invalid_argument("attention width must be a multiple of 8");
+    DecodeWorkspace ws;
+    ws.attach_workspace(p, input.device());
     hip_check(dlk_gemv(&p, context.stream), "attention QKV");
 
     dlk_attention_params a{};
@@ -284,6 +288,7 @@ Tensor GroupedQueryAttention::run(const Tensor& input, KVCache* cache) {
     o.ldy = d;
     o.bump_position = target.position_data();
     o.bump_count = L;
+    ws.attach_workspace(o, input.device());
     hip_check(dlk_gemv(&o, context.stream), "attention output");
     target.advance(L);
     return out;

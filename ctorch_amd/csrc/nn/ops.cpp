@@ -1,6 +1,6 @@
 // Decode-path operators on GPU tensors (reference include/dl/ops.h:100-101,149-158,191,341 and their
 // numeric layer, src/ops/numeric.cpp:178-226,252-254).  Low-precision inputs compute and return f32.
-#include "nn/ops_internal.h"
+#include "nn/decode_step.h"
 
 #include <algorithm>
 #include <cmath>
@@ -68,6 +68,8 @@ void linear_into(const float* x, Index rows, Index k, const Tensor& weight, cons
     p.w_bf16 = wb;
     p.y = y;
     p.ldy = ldy;
+    DecodeWorkspace ws; // released to the pool in stream order
+    ws.attach_workspace(p, weight.device());
     if (bias) {
         const Tensor b = bias->is_contiguous() ? *bias : bias->contiguous();
         if (b.dtype() != DType::f32 && b.dtype() != DType::bf16) throw std::invalid_argument("linear: bias dtype");
