@@ -2,9 +2,11 @@
 
 #include "dl/gpu.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <stdexcept>
 #include <vector>
 
@@ -66,14 +68,88 @@ void require_gpu(Device device, const char* operation) {
                                     ": this build computes on the GPU only; move the tensors/modules with to(gpu)");
 }
 
+namespace {
+
+bool capturing(const GpuContext& context) {
+    int active = 0;
+    hip_check(dlh_stream_capturing(context.stream, &active), "stream capture status");
+    return active != 0;
+}
+
+// returns the oldest blocks to the runtime's pool until at most `bytes` are held (the cache's mutex held)
+void shrink(GpuContext& context, std::size_t bytes, std::size_t blocks) {
+    auto& cache = context.cache;
+    while (cache.held > bytes || cache.blocks.size() > blocks) {
+        auto oldest = cache.blocks.begin();
+        for (auto it = cache.blocks.begin(); it != cache.blocks.end(); ++it)
+            if (it->second.age < oldest->second.age) oldest = it;
+        (void)dlh_free_async(oldest->second.data, context.stream);
+        cache.held -= oldest->first;
+        cache.blocks.erase(oldest);
+    }
+}
+
+// a block of at least `bytes`, which receives its size
+void* take_block(GpuContext& context, std::size_t& bytes) {
+    auto& cache = context.cache;
+    const bool direct = bytes > BlockCache::kBlockMax || capturing(context);
+    std::lock_guard<std::mutex> lock(cache.mutex);
+    void* data = nullptr;
+    if (!direct) {
+        // the smallest that fits, if at most an eighth of it goes unused
+        const auto found = cache.blocks.lower_bound(bytes);
+        if (found != cache.blocks.end() && found->first <= bytes + bytes / 8) {
+            bytes = found->first;
+            data = found->second.data;
+            cache.held -= bytes;
+            cache.blocks.erase(found);
+        }
+    }
+    if (!data) {
+        int status = dlh_malloc_async(&data, bytes, context.stream);
+        if (status != 0 && !direct && cache.held > 0) { // short of memory: the held blocks go back first
+            (void)dlh_last_launch_error();
+            shrink(context, 0, 0);
+            status = dlh_malloc_async(&data, bytes, context.stream);
+        }
+        hip_check(status, "allocate");
+    }
+    cache.live += bytes;
+    cache.peak = std::max(cache.peak, cache.live);
+    return data;
+}
+
+void give_block(GpuContext& context, void* data, std::size_t bytes) {
+    auto& cache = context.cache;
+    int active = 0;
+    const bool direct = bytes > BlockCache::kBlockMax || dlh_stream_capturing(context.stream, &active) != 0 || active != 0;
+    std::lock_guard<std::mutex> lock(cache.mutex);
+    cache.live -= bytes;
+    bool kept = false;
+    if (!direct && bytes <= cache.limit) {
+        try { // called from a destructor
+            cache.blocks.emplace(bytes, BlockCache::Block{data, cache.clock++});
+            kept = true;
+        } catch (const std::bad_alloc&) {
+        }
+    }
+    if (!kept) {
+        (void)dlh_free_async(data, context.stream);
+        return;
+    }
+    cache.held += bytes;
+    shrink(context, cache.limit, BlockCache::kBlocks);
+}
+
+} // namespace
+
 Storage::~Storage() {
     if (!data) return;
     if (device.type == DeviceType::cpu) {
         std::free(data);
     } else {
         // stream-ordered release: later work on the compute stream may reuse the block immediately
-        GpuContext& context = gpu_context(device.index);
-        (void)dlh_free_async(data, context.stream);
+        give_block(gpu_context(device.index), data, block);
     }
 }
 
@@ -87,8 +163,8 @@ std::shared_ptr<Storage> allocate_storage(std::size_t bytes, Device device) {
         if (!storage->data) throw std::bad_alloc();
         std::memset(storage->data, 0, rounded);
     } else {
-        GpuContext& context = gpu_context(device.index);
-        hip_check(dlh_malloc_async(&storage->data, rounded, context.stream), "allocate");
+        storage->block = rounded;
+        storage->data = take_block(gpu_context(device.index), storage->block);
     }
     return storage;
 }
@@ -117,26 +193,44 @@ void synchronize(Device device) {
 
 namespace dl::gpu {
 MemoryStats memory_stats(int device) {
-    detail::gpu_context(device);
+    auto& cache = detail::gpu_context(device).cache;
+    std::lock_guard<std::mutex> lock(cache.mutex);
     MemoryStats out{};
     detail::hip_check(dlh_pool_stats(device, &out.used_bytes, &out.reserved_bytes, &out.peak_used_bytes,
                                      &out.peak_reserved_bytes, &out.release_threshold),
                       "pool statistics");
+    // held blocks are free ones: `used` counts the live tensors and what others have of the pool
+    const std::uint64_t ours = cache.live + cache.held, others = out.used_bytes > ours ? out.used_bytes - ours : 0;
+    out.used_bytes = cache.live + others;
+    out.peak_used_bytes = cache.peak > 0 ? cache.peak + others : 0;
     return out;
 }
 
 void set_memory_release_threshold(std::uint64_t bytes, int device) {
-    detail::gpu_context(device);
+    auto& context = detail::gpu_context(device);
+    {
+        std::lock_guard<std::mutex> lock(context.cache.mutex);
+        context.cache.limit = static_cast<std::size_t>(std::min<std::uint64_t>(bytes, detail::BlockCache::kLimit));
+        detail::shrink(context, context.cache.limit, detail::BlockCache::kBlocks);
+    }
     detail::hip_check(dlh_pool_set_threshold(device, bytes), "pool release threshold");
 }
 
 void reset_peak_memory_stats(int device) {
-    detail::gpu_context(device);
+    auto& cache = detail::gpu_context(device).cache;
+    {
+        std::lock_guard<std::mutex> lock(cache.mutex);
+        cache.peak = 0; // the next allocation raises it again
+    }
     detail::hip_check(dlh_pool_reset_peaks(device), "pool peak reset");
 }
 
 void release_unused_memory(int device) {
     auto& context = detail::gpu_context(device);
+    {
+        std::lock_guard<std::mutex> lock(context.cache.mutex);
+        detail::shrink(context, 0, 0);
+    }
     detail::hip_check(dlh_stream_synchronize(context.stream), "synchronize");
     detail::hip_check(dlh_pool_trim(device), "pool trim");
 }
