@@ -76,13 +76,14 @@ inline int64_t blocks_of(const dlk_gemv_params& p, int shape) {
 /// 2000 x 4096 -> 16000: 2718 (2000) / 2912 / 3124 / 3805;  500 x 2048 -> 8191: 216 (256) / 217 (1024) / 234 / 293;
 /// 300 x 2048 -> 16000: 345 (375) / 243 (1250) / 265 / 308;  2040 x 256 -> 1376: 30.1 (176) / 24.2 (704) / 25.5 / 34.9;
 /// 150 x 2048 -> 16000: 189 / 150 (750) / 137 (1250) / 162;  300 x 4096 -> 4000: 367 / 214 (315) / 182 (630) / 176.
-/// With fewer work-groups than that a launch is a chain of chunk round trips, and waves that split the k make the
+/// 2040 x 688 -> 256 (64x32: 256) 16.9 against 17.8, and with the norm's sums in every column block 256 -> 384 (384) 14.1
+/// against 16.8.  With fewer work-groups than that a launch is a chain of chunk round trips, and waves that split the k make the
 /// chain four times shorter: 510 x 688 -> 256: 64.9 / 22.4 / 16.4 (64) / 7.7 (256);  34 x 256 -> 1376: 25.7 / 10.7 / 7.8 /
 /// 4.7;  9 x 4096 -> 250: 356 / 116 / 79 / 25.
 inline int shape_of(const dlk_gemv_params& p) {
     if (blocks_of(p, k128x128) >= 1024) return k128x128;
     if (blocks_of(p, k64x64) >= 512) return k64x64;
-    if (blocks_of(p, k64x32) >= 512) return k64x32;
+    if (blocks_of(p, k64x32) >= 256) return k64x32;
     return k32x16;
 }
 
