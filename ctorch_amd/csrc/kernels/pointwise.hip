@@ -175,13 +175,39 @@ __global__ void rope_kernel(const float* x, int64_t outer, int64_t length, int64
     }
 }
 
-// Greedy or Gumbel-max candidates: block (row, part) scans a contiguous slice of the row.
+// The Gumbel noise of sample_score to within 1e-4, in f32: a bound that tells which entries cannot be the best.  The
+// logarithm near one is taken from 1 - u, whose bits are exact (2 atanh series), and the rest is the hardware's log2.
+__device__ __forceinline__ float gumbel_about(uint64_t seed, uint64_t stream, uint64_t index) {
+    uint32_t b[4];
+    philox(seed, index, stream, b);
+    const uint64_t half = ((static_cast<uint64_t>(b[0] >> 5) << 26) | (b[1] >> 6)) >> 1; // u = (half + 1/2) 2^-52
+    constexpr uint64_t kOne = uint64_t(1) << 52;
+    float w; // -log u, to a relative 1e-5
+    if (half >= kOne / 2) {
+        const float v = (static_cast<float>(kOne - 1 - half) + 0.5f) * 0x1p-52f; // 1 - u, at most 1/2
+        const float s = v / (2.0f - v), t = s * s;                                // at most 1/3
+        w = 2.0f * s * (1.0f + t * (1.0f / 3 + t * (1.0f / 5 + t * (1.0f / 7 + t * (1.0f / 9)))));
+    } else {
+        w = -0.6931471805599453f * __builtin_amdgcn_logf((static_cast<float>(half) + 0.5f) * 0x1p-52f);
+    }
+    return -0.6931471805599453f * __builtin_amdgcn_logf(w);
+}
+
+// Greedy or Gumbel-max candidates: block (row, part) scans a contiguous slice of the row.  Sampling scores take two
+// portable double logarithms an entry, some 250 double instructions.  So the scores are first computed in f32 (two
+// hardware logarithms), and only the entries that could still be the best of the slice, given what f32 may be off by,
+// are evaluated in double; the largest exact score is among them.  The noise error is below 1e-4 (derived at
+// gumbel_about, with the logarithm's 1e-6 on |g| <= 37), the scaled logit's below 2^-22 of itself; the margin is ten
+// times that.  Bound by the Philox rounds.  Measured on MI355X, 32 x 32000 logits:
+// 15.3 -> 9.1 us.
+constexpr int kSamplePer = 8; // entries per thread held between the two passes (slices of at most 2048)
 __global__ __launch_bounds__(kThreads) void sample_partials_kernel(const float* logits, int64_t n, int mode,
                                                                    double temperature, uint64_t key_seed,
                                                                    uint64_t key_stream, const int64_t* key_label,
                                                                    dlk_sample_partial* partial, int blocks) {
     __shared__ double best_score[kThreads];
     __shared__ int64_t best_index[kThreads];
+    __shared__ float wave_least[kThreads / kWave];
     const int64_t row = blockIdx.y;
     const int part = blockIdx.x;
     uint64_t seed = key_seed, stream = key_stream;
@@ -190,10 +216,35 @@ __global__ __launch_bounds__(kThreads) void sample_partials_kernel(const float* 
     const int64_t begin = part * per, end = min(n, begin + per);
     double best = 0.0;
     int64_t index = -1;
-    for (int64_t i = begin + threadIdx.x; i < end; i += kThreads) {
+    auto consider = [&](int64_t i) {
         const double s = sample_score(logits[row * n + i], mode, temperature, seed, stream,
                                       static_cast<uint64_t>(row * n + i));
         if (index < 0 || prefer(s, i, best, index)) { best = s; index = i; }
+    };
+    const float inverse = static_cast<float>(1.0 / temperature);
+    if (mode == 2 && per <= kSamplePer * kThreads && inverse > 1e-30f && inverse < 1e30f) {
+        float about[kSamplePer], margin[kSamplePer];
+        float least = -INFINITY; // the largest score that some entry certainly reaches
+#pragma unroll
+        for (int j = 0; j < kSamplePer; ++j) {
+            const int64_t i = begin + threadIdx.x + j * kThreads;
+            const float scaled = logits[row * n + min(i, end - 1)] * inverse;
+            about[j] = scaled + gumbel_about(seed, stream, static_cast<uint64_t>(row * n + min(i, end - 1)));
+            margin[j] = fabsf(scaled) < INFINITY ? 1e-3f + fabsf(scaled) * 2.4e-6f : 0.0f;
+            if (i < end) least = fmaxf(least, about[j] - margin[j]); // a NaN is left out here and evaluated below
+        }
+        least = wave_max(least);
+        if (threadIdx.x % kWave == 0) wave_least[threadIdx.x / kWave] = least;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kThreads / kWave; ++w) least = fmaxf(least, wave_least[w]);
+#pragma unroll
+        for (int j = 0; j < kSamplePer; ++j) {
+            const int64_t i = begin + threadIdx.x + j * kThreads;
+            if (i < end && !(about[j] + margin[j] < least)) consider(i);
+        }
+    } else {
+        for (int64_t i = begin + threadIdx.x; i < end; i += kThreads) consider(i);
     }
     best_score[threadIdx.x] = best;
     best_index[threadIdx.x] = index;

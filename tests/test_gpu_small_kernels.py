@@ -1,4 +1,5 @@
-"""RMSNorm over every width class, against 64-bit results."""
+"""Sampling from logits that bound or break its f32 pre-selection, and RMSNorm over every width class, against the
+oracle (sampling bit for bit)."""
 import numpy as np
 import pytest
 
@@ -8,6 +9,34 @@ from common import say
 
 pytestmark = pytest.mark.gpu
 GPU = ct.device("gpu")
+
+
+@pytest.mark.parametrize("vocab", [1, 3, 2048, 2049, 32000, 131072, 131073])
+@pytest.mark.parametrize("temperature", [0.05, 0.8, 1.0, 40.0])
+def test_sampling_is_bit_exact_whatever_the_logits_hold(vocab, temperature):
+    say(f"case: dl_sample, vocab {vocab}, temperature {temperature}")
+    rng = np.random.default_rng(vocab)
+    rows = np.empty((9, vocab), np.float32)
+    rows[:] = 3 * rng.standard_normal((9, vocab))
+    rows[1] = 0.0                                               # the noise decides
+    rows[2, rng.random(vocab) < 0.9] = -np.inf                  # masked entries
+    rows[3] = -np.inf
+    rows[4, vocab // 2] = np.inf
+    rows[5, [vocab - 1, vocab // 3]] = np.nan
+    rows[6] *= 1e37                                             # the scaled logits overflow f32
+    rows[7] = np.float32(1e30) + np.zeros(vocab, np.float32)    # the noise is lost in the logits: ties
+    rows[8] *= 1e-30
+    for key in ((1, 2), (2**64 - 1, 77)):
+        got = ct.sample(ct.Tensor.from_numpy(rows, ct.F32, GPU), temperature, key).numpy()
+        assert np.array_equal(got, oracle.sample(rows, temperature, key)), key
+
+
+def test_sampling_at_temperatures_beyond_f32():
+    say("case: dl_sample at temperatures whose inverse f32 cannot hold")
+    rows = np.random.default_rng(8).standard_normal((3, 5000)).astype(np.float32)
+    for temperature in (1e-45, 1e-35, 1e35, 1e300):
+        got = ct.sample(ct.Tensor.from_numpy(rows, ct.F32, GPU), temperature, (5, 6)).numpy()
+        assert np.array_equal(got, oracle.sample(rows, temperature, (5, 6))), temperature
 
 
 @pytest.mark.parametrize("width", [1, 4, 6, 1000, 1024, 1028, 2048, 4100, 8192, 8196])
