@@ -22,7 +22,7 @@
 // 4 sequences x 7 positions over 1508 f32 keys, 32 / 8 heads of 64: 135.5 -> 11.6 us + 4.7 for the merge; 4 x 500
 // positions bidirectional over a padded batch: 455 -> 107 us (the products alone take 38; exponentials, masks and staging
 // as much vector work again, and the two barriers of a tile keep them from overlapping fully); causal byte prompts of
-// 4 x 510 positions, 8 / 2 heads of 32: 84 -> 18 us; one position of that model over 160 keys: 5.7 -> 5.1 us.
+// 4 x 510 positions, 8 / 2 heads of 32: 84 -> 15 us; one position of that model over 160 keys: 5.7 -> 5.1 us.
 #include "kernels/device_common.h"
 
 #include <algorithm>
@@ -484,7 +484,11 @@ int launch_combine(const dlk_attention_params& p, hipStream_t stream) {
 template <typename KT, int HD>
 int launch(const dlk_attention_params& p, hipStream_t stream) {
     const int rows = p.H / p.KV * p.L;
-    const int wr = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+    int wr = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+    // four row tiles that leave a CU with less than two work-groups: two, so that one's products run under another's
+    // staging and softmax (4 x 510 causal positions, 8 / 2 heads of 32: 18.5 us at 256 work-groups, 15.2 at 512, 16.8 at
+    // 1024 of one row tile; 4 x 500 positions of 32 / 8 heads of 64: 111 at 1024, 120 at 2048)
+    if (wr == 4 && static_cast<int64_t>((rows + 63) / 64) * p.splits * p.B * p.KV < 512) wr = 2;
     const dim3 grid(p.splits, (rows + 16 * wr - 1) / (16 * wr), p.B * p.KV);
     const dim3 threads(kThreads);
     if (wr == 1) hipLaunchKernelGGL((attention_rows<KT, HD, 1>), grid, threads, 0, stream, p);
