@@ -20,7 +20,7 @@
 // What bounds it: many rows, the f32 matrix cores (153 TFLOP/s); few rows, the round trips of the K/V tiles.
 // Measured on MI355X (the kernel before it ran the products on the vector ALU, one key or head-dim column per lane):
 // 4 sequences x 7 positions over 1508 f32 keys, 32 / 8 heads of 64: 135.5 -> 11.6 us + 4.7 for the merge; 4 x 500
-// positions bidirectional over a padded batch: 455 -> 107 us (the products alone take 38; exponentials, masks and staging
+// positions bidirectional over a padded batch: 455 -> 90 us (the products alone take 38; exponentials, masks and staging
 // as much vector work again, and the two barriers of a tile keep them from overlapping fully); causal byte prompts of
 // 4 x 510 positions, 8 / 2 heads of 32: 84 -> 15 us; one position of that model over 160 keys: 5.7 -> 5.1 us.
 #include "kernels/device_common.h"
@@ -66,14 +66,17 @@ __global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_p
 
     const int t = threadIdx.x, lane = t % kWave, q = lane / 16, r = lane % 16;
     const int wave = __builtin_amdgcn_readfirstlane(t / kWave), wr = wave / WK, wk = wave % WK;
-    // consecutive work-group ids go to the 8 XCDs in turn: each XCD takes a run of the order in which the splits and
-    // row blocks of a KV head are neighbours, so its L2 holds the few KV heads it works on
-    const int total = gridDim.x * gridDim.y * gridDim.z;
+    // Consecutive work-group ids go to the 8 XCDs in turn.  With the (sequence, KV head) pairs a multiple of 8, XCD x takes
+    // the splits and row blocks of pairs x, x + 8, ... one pair after the other, so its L2 holds the few pairs it works
+    // on and the sequences of a padded batch, whose masks leave them different work, spread over all XCDs (each XCD
+    // on a sequence of its own: 4 x 500 positions 111 -> 90 us).  Otherwise each takes a run of the pairs.
+    const int per_pair = gridDim.x * gridDim.y, total = per_pair * gridDim.z;
     const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = id % 8, per = total / 8, rem = total % 8;
-    const int logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + id / 8;
+    const int xcd = id % 8, idx = id / 8, per = total / 8, rem = total % 8;
+    const int logical = gridDim.z % 8 == 0 ? (idx / per_pair * 8 + xcd) * per_pair + idx % per_pair
+                                           : (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
     const int split = logical % gridDim.x, row_block = logical / gridDim.x % gridDim.y;
-    const int pair = logical / (gridDim.x * gridDim.y);
+    const int pair = logical / per_pair;
     const int b = pair / p.KV, kvh = pair % p.KV;
     const int G = p.H / p.KV;
     const int rows_total = G * p.L, row0 = row_block * 16 * WR;
