@@ -76,6 +76,16 @@ inline bool repacked(const dlk_gemv_params& p) {
     return true;
 }
 
+/// 16 bytes of weights.  Repacked weights (every launch of the deep pipeline, which is compiled for them alone)
+/// stream past the caches: a load instruction of a wave takes whole lines, once.  Of row-major weights it takes
+/// 64 bytes of each of 16 rows, half a line, and the next step's load the other half: those stay cached in between.
+template <bool REPACKED>
+__device__ __forceinline__ u32x4 load_weights(const uint16_t* w, bool repacked) {
+    const u32x4* src = reinterpret_cast<const u32x4*>(w);
+    if (REPACKED || repacked) return __builtin_nontemporal_load(src);
+    return *src;
+}
+
 /// 16-row weight tiles of a launch.
 __host__ __device__ inline int tiles_of(const dlk_gemv_params& p) {
     if (p.epilogue == DLK_EPI_SWIGLU) return p.seg_rows[0] / 8;
@@ -448,8 +458,7 @@ __global__ __launch_bounds__(kThreads) void gemm_rows(const dlk_gemv_params laun
     auto load_w = [&](int c, u32x4 (&dst)[STEPS]) {
 #pragma unroll
         for (int s = 0; s < STEPS; ++s)
-            dst[s] = __builtin_nontemporal_load(
-                reinterpret_cast<const u32x4*>(wsrc + c * chunk_stride + s * step_stride));
+            dst[s] = load_weights<(NC >= 4)>(wsrc + c * chunk_stride + s * step_stride, wtiles != nullptr);
     };
     f32x4 acc[MT];
 #pragma unroll
