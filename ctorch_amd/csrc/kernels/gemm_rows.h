@@ -13,7 +13,7 @@
 // (NC = 2) issues every activation and weight load of its chunks at once, stages them all, and computes: one
 // memory round trip.  Longer runs double buffer the chunks in LDS: with repacked weights and a run of 4, 8, 16 or
 // 32 chunks (NC = the run) the weights of the next three chunks are in flight while one is used; otherwise
-// (NC = 0) the next chunk's activations (into registers) and weights.
+// (NC = 0 with repacked weights, 1 with row-major ones) the next chunk's activations (into registers) and weights.
 //
 // Tile rows: generic epilogues take 16 consecutive rows of one weight segment; SwiGLU interleaves gate and up
 // (tile row 2j = gate row 8T + j, 2j + 1 = up row 8T + j), so every lane holds (gate, up) pairs and QKV holds
@@ -45,16 +45,16 @@ constexpr size_t lds_bytes(int mt) { return size_t(2) * 2 * 16 * mt * lds_stride
 /// 3 ahead 1.183 ms; 4 (16-row tiles) / 6 (32-row tiles) ahead 1.198-1.210 ms; 5 / 8 ahead 1.214-1.225 ms.
 constexpr int kDeepAhead = 3;
 /// Variant for a run of `nchunks` chunks: 2 (all loads up front; that many chunks at most), the run length itself
-/// (the deep pipeline, unrolled over a run of 4, 8, 16 or 32 chunks; `deep`: repacked weights and 16 or more
-/// activation rows per work-group), or 0 for the double-buffered loop.  Measured on MI355X (A/B, one box): at batch
-/// 32 (1B) the deep pipeline took the C3 step 1.190-1.204 -> 1.168-1.170 ms (gate/up 15.5 -> 14.9 us, down 11.7-12.2
+/// (the deep pipeline, unrolled over a run of 4, 8, 16 or 32 chunks of repacked weights; `deep`: 16 or more
+/// activation rows per work-group), or the double-buffered loop (0: repacked weights, 1: row-major ones, see
+/// load_weights).  Measured on MI355X (A/B, one box): at batch 32 (1B) the deep pipeline took the C3 step 1.190-1.204 -> 1.168-1.170 ms (gate/up 15.5 -> 14.9 us, down 11.7-12.2
 /// -> 10.9, LM head 30.5-31.1 -> 29.3); at 8 rows (8B, batch 8) the QKV and gate/up launches, already streaming at
 /// ~5.6 TB/s, lost 1-1.7 us each, so those keep the loop.  Runs of three or four chunks take a loop, not all loads
 /// up front (C3 down projection in 11 key slices of 4 chunks: 11.2 us a layer against 12.7).
-constexpr int loop_variant(int nchunks, bool deep) {
+constexpr int loop_variant(int nchunks, bool repacked, bool deep) {
     if (nchunks <= 2) return 2;
-    if (deep && (nchunks == 4 || nchunks == 8 || nchunks == 16 || nchunks == 32)) return nchunks;
-    return 0;
+    if (repacked && deep && (nchunks == 4 || nchunks == 8 || nchunks == 16 || nchunks == 32)) return nchunks;
+    return repacked ? 0 : 1;
 }
 /// Most key slices a launch takes (the reduce kernel keeps them all in flight).
 constexpr int kMaxSplits = 16;
@@ -76,14 +76,17 @@ inline bool repacked(const dlk_gemv_params& p) {
     return true;
 }
 
-/// 16 bytes of weights.  Repacked weights (every launch of the deep pipeline, which is compiled for them alone)
-/// stream past the caches: a load instruction of a wave takes whole lines, once.  Of row-major weights it takes
-/// 64 bytes of each of 16 rows, half a line, and the next step's load the other half: those stay cached in between.
-template <bool REPACKED>
-__device__ __forceinline__ u32x4 load_weights(const uint16_t* w, bool repacked) {
+/// 16 bytes of weights, for loop variant NC.  Repacked weights stream past the caches: a load instruction of a wave
+/// takes whole lines, once.  Of row-major weights it takes 64 bytes of each of 16 rows, half a line, and the next
+/// step's load the other half, so their loop (NC = 1) keeps the line cached in between.  Measured on MI355X (8B
+/// widths, 8 rows): gate/up 53.3 -> 44.3 us (5.3 TB/s), O and down 17.5 -> 15.8, QKV 15.2 -> 13.9; a 1B check of 16
+/// drafted tokens 313 -> 291 us.  The variant is a template because choosing by a branch at the loads cost the
+/// repacked loop 2 % of an 8B decode step at batch 8 (9.38 -> 9.55 ms).
+template <int NC>
+__device__ __forceinline__ u32x4 load_weights(const uint16_t* w) {
     const u32x4* src = reinterpret_cast<const u32x4*>(w);
-    if (REPACKED || repacked) return __builtin_nontemporal_load(src);
-    return *src;
+    if constexpr (NC == 1) return *src;
+    else return __builtin_nontemporal_load(src);
 }
 
 /// 16-row weight tiles of a launch.
@@ -458,7 +461,7 @@ __global__ __launch_bounds__(kThreads) void gemm_rows(const dlk_gemv_params laun
     auto load_w = [&](int c, u32x4 (&dst)[STEPS]) {
 #pragma unroll
         for (int s = 0; s < STEPS; ++s)
-            dst[s] = load_weights<(NC >= 4)>(wsrc + c * chunk_stride + s * step_stride, wtiles != nullptr);
+            dst[s] = load_weights<NC>(wsrc + c * chunk_stride + s * step_stride);
     };
     f32x4 acc[MT];
 #pragma unroll
@@ -986,6 +989,7 @@ gemv::Kernel resolve(const dlk_gemv_params& p, int mt, int nc) {
             constexpr int MT = decltype(mtc)::value;
             switch (nc) {
             case 0: return DLK_GEMM_ROWS(MT, 0);
+            case 1: return DLK_GEMM_ROWS(MT, 1);
             case 2: return DLK_GEMM_ROWS(MT, 2);
             case 4: return DLK_GEMM_ROWS(MT, 4);
             case 8: return DLK_GEMM_ROWS(MT, 8);

@@ -193,7 +193,7 @@ int launch_gemm(const dlk_gemv_params& params, hipStream_t stream) {
         if (p.epilogue == DLK_EPI_SWIGLU && parts > 1 && blocks >= 64 && blocks * parts <= 256 && blocks % 8 == 0) {
             p.row_parts = parts;
             // parts of 16 rows: the deep pipeline when the weights come repacked
-            const Kernel kernel = resolve_gemm(p, 1, loop_variant(p.K / chunk_k(1), repacked(p)));
+            const Kernel kernel = resolve_gemm(p, 1, loop_variant(p.K / chunk_k(1), repacked(p), true));
             if (!kernel.fn) return static_cast<int>(hipErrorInvalidValue);
             void* args[] = {&p};
             const hipError_t status =
@@ -211,8 +211,7 @@ int launch_gemm(const dlk_gemv_params& params, hipStream_t stream) {
         if (p.defer_reduce && (splits == 1 || p.epilogue != DLK_EPI_QKV || params.M > kMaxRows))
             return static_cast<int>(hipErrorInvalidValue);
         const int mt = row_tiles(p.M);
-        const bool deep = repacked(p) && p.M >= 16;
-        const Kernel kernel = resolve_gemm(p, mt, loop_variant(p.K / splits / chunk_k(mt), deep));
+        const Kernel kernel = resolve_gemm(p, mt, loop_variant(p.K / splits / chunk_k(mt), repacked(p), p.M >= 16));
         if (!kernel.fn) return static_cast<int>(hipErrorInvalidValue);
         const int64_t* bump = p.bump_position;
         if (splits > 1) p.bump_position = nullptr; // the reduce launch advances the length
