@@ -68,8 +68,10 @@ void linear_into(const float* x, Index rows, Index k, const Tensor& weight, cons
     p.w_bf16 = wb;
     p.y = y;
     p.ldy = ldy;
-    DecodeWorkspace ws; // released to the pool in stream order
-    ws.attach_workspace(p, weight.device());
+    // the workspace of the staged kernels (released to the pool in stream order), as large as the rows: past 4 GiB of
+    // rows the launches of 64 rows, which need none, keep a product that fits the card only without it
+    DecodeWorkspace ws;
+    if (rows * k <= (Index{1} << 30)) ws.attach_workspace(p, weight.device());
     if (bias) {
         const Tensor b = bias->is_contiguous() ? *bias : bias->contiguous();
         if (b.dtype() != DType::f32 && b.dtype() != DType::bf16) throw std::invalid_argument("linear: bias dtype");

@@ -50,12 +50,33 @@ def test_attention_rows_match_64_bit_results(B, H, KV, L, S, D, bf16, masked):
         gm = None if mask is None else ct.Tensor.from_numpy(mask, ct.BOOL, GPU)
         want = reference(q, k, v, mask)
         assert np.isnan(want).any() == nan
-        # the query as stored, and as a [B, L, H, D] tensor's transposed view would be made contiguous by the caller
         got = ct.grouped_query_attention(ct.Tensor.from_numpy(q, ct.F32, GPU), gk, gv, gm).numpy()
         assert np.array_equal(np.isnan(got), np.isnan(want))
         # f32 sums: a score is off by some |score| 2^-24 sqrt(D), a weighted sum by 2^-24 sqrt(S)
         error = np.nan_to_num(got - want)
         assert np.linalg.norm(error) <= 2.0**-24 * (np.sqrt(D) + np.sqrt(S) + 8) * np.linalg.norm(np.nan_to_num(want))
+
+
+@pytest.mark.parametrize("L,S,masked", [(5, 130, False), (5, 130, True), (1, 70, True), (70, 90, False)])
+@pytest.mark.parametrize("axis,start", [(0, 1), (1, 2), (2, 1), (3, 1)])
+def test_views_of_a_query_and_a_mask_are_read_through_their_strides(L, S, masked, axis, start):
+    say(f"case: attention, query narrowed along axis {axis} from {start}, L={L} S={S} masked={masked}")
+    rng = np.random.default_rng(axis + S)
+    shape = [2, 4, L, 32]
+    view = lambda t, a, s, n: ct.Tensor(ct._new(ct.lib().dl_narrow, t.handle, a, s, n))
+    stored = [n + (start + 1) * (i == axis) for i, n in enumerate(shape)]  # axis 3 from 1: rows off the 16-byte grid
+    q = rng.standard_normal(stored).astype(np.float32)
+    k, v = (rng.standard_normal((2, 2, S, 32)).astype(np.float32) for _ in range(2))
+    gq = view(ct.Tensor.from_numpy(q, ct.F32, GPU), axis, start, shape[axis])
+    gm = keep = None
+    if masked:
+        wide = rng.random((2, 1, L, S + 3)) < 0.6
+        wide[..., 3] = True
+        keep, gm = wide[..., 3:], view(ct.Tensor.from_numpy(wide, ct.BOOL, GPU), 3, 3, S)
+    got = ct.grouped_query_attention(gq, *(ct.Tensor.from_numpy(a, ct.F32, GPU) for a in (k, v)), gm).numpy()
+    q = np.take(q, range(start, start + shape[axis]), axis)
+    want = reference(q, k, v, keep)
+    assert np.linalg.norm(got - want) <= 2.0**-24 * (np.sqrt(32) + np.sqrt(S) + 8) * np.linalg.norm(want)
 
 
 @pytest.mark.parametrize("bf16", [False, True])
