@@ -92,7 +92,7 @@ void shrink(GpuContext& context, std::size_t bytes, std::size_t blocks) {
 // a block of at least `bytes`, which receives its size
 void* take_block(GpuContext& context, std::size_t& bytes) {
     auto& cache = context.cache;
-    const bool direct = bytes > BlockCache::kBlockMax || capturing(context);
+    const bool captured = capturing(context), direct = captured || bytes > BlockCache::kBlockMax;
     std::lock_guard<std::mutex> lock(cache.mutex);
     void* data = nullptr;
     if (!direct) {
@@ -107,7 +107,7 @@ void* take_block(GpuContext& context, std::size_t& bytes) {
     }
     if (!data) {
         int status = dlh_malloc_async(&data, bytes, context.stream);
-        if (status != 0 && !direct && cache.held > 0) { // short of memory: the held blocks go back first
+        if (status != 0 && !captured && cache.held > 0) { // short of memory: the held blocks go back first
             (void)dlh_last_launch_error();
             shrink(context, 0, 0);
             status = dlh_malloc_async(&data, bytes, context.stream);
