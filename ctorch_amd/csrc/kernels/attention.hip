@@ -20,9 +20,10 @@
 // What bounds it: many rows, the f32 matrix cores (153 TFLOP/s); few rows, the round trips of the K/V tiles.
 // Measured on MI355X (the kernel before it ran the products on the vector ALU, one key or head-dim column per lane):
 // 4 sequences x 7 positions over 1508 f32 keys, 32 / 8 heads of 64: 135.5 -> 11.6 us + 4.7 for the merge; 4 x 500
-// positions bidirectional over a padded batch: 455 -> 90 us (the products alone take 38; exponentials, masks and staging
+// positions bidirectional over a padded batch: 455 -> 85 us (the products alone take 38; exponentials, masks and staging
 // as much vector work again, and the two barriers of a tile keep them from overlapping fully); causal byte prompts of
-// 4 x 510 positions, 8 / 2 heads of 32: 84 -> 15 us; one position of that model over 160 keys: 5.7 -> 5.1 us.
+// 4 x 510 positions, 8 / 2 heads of 32: 84 -> 15 us; one position of that model: 5.7 -> 5.0 us (4.6 up to 128 keys; each
+// further tile is a round trip of 1.7 us).
 #include "kernels/device_common.h"
 
 #include <algorithm>
@@ -50,7 +51,7 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 template <typename KT, int HD, int WR>
-__global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_params p) {
+__global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_params p, int G) {
     constexpr int WK = kWaves / WR;                   // waves that share a row tile's keys
     constexpr int T = tile_keys(HD, WR);
     constexpr int GROUPS = T / 16 / WK;               // 16-key groups of a tile per wave
@@ -70,15 +71,21 @@ __global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_p
     // the splits and row blocks of pairs x, x + 8, ... one pair after the other, so its L2 holds the few pairs it works
     // on and the sequences of a padded batch, whose masks leave them different work, spread over all XCDs (each XCD
     // on a sequence of its own: 4 x 500 positions 111 -> 90 us).  Otherwise each takes a run of the pairs.
-    const int per_pair = gridDim.x * gridDim.y, total = per_pair * gridDim.z;
-    const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = id % 8, idx = id / 8, per = total / 8, rem = total % 8;
-    const int logical = gridDim.z % 8 == 0 ? (idx / per_pair * 8 + xcd) * per_pair + idx % per_pair
-                                           : (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
-    const int split = logical % gridDim.x, row_block = logical / gridDim.x % gridDim.y;
-    const int pair = logical / per_pair;
-    const int b = pair / p.KV, kvh = pair % p.KV;
-    const int G = p.H / p.KV;
+    // One work-group a pair has nothing to share: it skips the divisions, a chain of some 300 instructions before its
+    // first load.  With those of the query row moved behind the first tile's loads, and the remainders replaced by
+    // products: one position of 8 / 2 heads of 32 over 33-160 keys 5.25 -> 4.98 us, the padded batch of 4 x 500 90 -> 85.
+    const int per_pair = gridDim.x * gridDim.y;
+    int split = 0, row_block = 0, pair = blockIdx.z;
+    if (per_pair > 1) {
+        const int total = per_pair * gridDim.z;
+        const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const int xcd = id % 8, idx = id / 8, per = total / 8, rem = total % 8;
+        const int logical = gridDim.z % 8 == 0 ? (idx / per_pair * 8 + xcd) * per_pair + idx % per_pair
+                                               : (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + idx;
+        split = logical % gridDim.x;
+        row_block = logical / gridDim.x % gridDim.y;
+        pair = logical / per_pair;
+    }
     const int rows_total = G * p.L, row0 = row_block * 16 * WR;
 
     const size_t head_base = static_cast<size_t>(pair) * p.capacity;
@@ -87,18 +94,28 @@ __global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_p
     const int64_t k_begin = static_cast<int64_t>(split) * p.chunk;
 
     const int64_t first = p.position ? *p.position : p.first_host;
-    // this lane's query row (rows past the end repeat the last; their results are never written)
-    const int row = min(row0 + 16 * wr + r, rows_total - 1);
-    const int l = row / G, h = kvh * G + row % G;
-    const unsigned char* keep =
-        p.keep_mask ? p.keep_mask + b * p.mask_stride[0] + h * p.mask_stride[1] + l * p.mask_stride[2] : nullptr;
 
     u32x4 k_next[LOADS], v_next[LOADS];
     uint32_t keep_next[GROUPS]; // four mask bytes each
-    // loads the tile's rows and this lane's mask entries; those from `end` on repeat the one before it and are dropped
-    // when the tile is used (the mask comes first: loads complete in order, and it would wait for the rows)
+    const unsigned char* keep = nullptr; // this lane's mask row
+    // load_tile loads the tile's rows and this lane's mask entries; those from `end` on repeat the one before it and are
+    // dropped when the tile is used (the mask comes first: loads complete in order, and it would wait for the rows)
+    auto load_rows = [&](int64_t tile0, int last) {
+        const KT* kt = kbase + tile0 * HD;
+        const KT* vt = vbase + tile0 * HD;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const int at = t + i * kThreads;
+            const uint32_t offset = min(at / PIECES, last) * HD + at % PIECES * VALUES;
+            k_next[i] = *reinterpret_cast<const u32x4*>(kt + offset);
+            v_next[i] = *reinterpret_cast<const u32x4*>(vt + offset);
+        }
+    };
+    auto last_of = [&](int64_t tile0, int64_t end) { // of the tile's rows, uniform
+        return static_cast<int>(min<int64_t>(end - tile0, T)) - 1;
+    };
     auto load_tile = [&](int64_t tile0, int64_t end) {
-        const int last = static_cast<int>(min<int64_t>(end - tile0, T)) - 1; // of the tile, uniform
+        const int last = last_of(tile0, end);
         if (keep) {
             const int64_t stride = p.mask_stride[3];
             const unsigned char* entries = keep + tile0 * stride;
@@ -117,20 +134,22 @@ __global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_p
                 }
             }
         }
-        const KT* kt = kbase + tile0 * HD;
-        const KT* vt = vbase + tile0 * HD;
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            const int at = t + i * kThreads;
-            const uint32_t offset = min(at / PIECES, last) * HD + at % PIECES * VALUES;
-            k_next[i] = *reinterpret_cast<const u32x4*>(kt + offset);
-            v_next[i] = *reinterpret_cast<const u32x4*>(vt + offset);
-        }
+        load_rows(tile0, last);
     };
-    // the first tile is requested before the device length arrives, within the storage: what lies past the length is
-    // dropped
+    // the first tile is requested before the device length arrives, and before the divisions below where no mask entry
+    // has to come first, within the storage: what lies past the length is dropped
     const int64_t stored = min(p.capacity, k_begin + p.chunk);
-    if (k_begin < stored) load_tile(k_begin, stored);
+    if (k_begin < stored && !p.keep_mask) load_rows(k_begin, last_of(k_begin, stored));
+
+    // this lane's query row (rows past the end repeat the last; their results are never written)
+    const int b = p.B == 1 ? 0 : pair / p.KV, kvh = pair - b * p.KV;
+    auto position_of = [&](int row) { return p.L == 1 ? 0 : row / G; };
+    const int row = min(row0 + 16 * wr + r, rows_total - 1);
+    const int l = position_of(row), h = kvh * G + row - l * G;
+    if (p.keep_mask) {
+        keep = p.keep_mask + b * p.mask_stride[0] + h * p.mask_stride[1] + l * p.mask_stride[2];
+        if (k_begin < stored) load_tile(k_begin, stored);
+    }
 
     const int64_t m_row = static_cast<int64_t>(b) * p.L + l;
     f32x4 qf[DT];
@@ -147,11 +166,11 @@ __global__ __launch_bounds__(kThreads) void attention_rows(const dlk_attention_p
     const int64_t limit = p.causal ? min(split_end, first + l + 1) : split_end;
     const int first_row = min(row0 + 16 * wr, rows_total - 1);
     const int last_row = min(row0 + 16 * wr + 15, rows_total - 1), last_block_row = min(row0 + 16 * WR - 1, rows_total - 1);
-    const int64_t wave_full = p.causal ? min(split_end, first + first_row / G + 1) : split_end;
+    const int64_t wave_full = p.causal ? min(split_end, first + position_of(first_row) + 1) : split_end;
     const int64_t wave_end = row0 + 16 * wr >= rows_total ? 0 // no row for this wave
-                             : p.causal                   ? min(split_end, first + last_row / G + 1)
+                             : p.causal                   ? min(split_end, first + position_of(last_row) + 1)
                                                           : split_end;
-    const int64_t k_end = p.causal ? min(split_end, first + last_block_row / G + 1) : split_end;
+    const int64_t k_end = p.causal ? min(split_end, first + position_of(last_block_row) + 1) : split_end;
 
     auto stage_tile = [&](int64_t tile0) {
         const int staged = static_cast<int>(min<int64_t>(k_end - tile0, T)); // live keys of the tile
@@ -486,7 +505,7 @@ int launch_combine(const dlk_attention_params& p, hipStream_t stream) {
 // The fewest row tiles per work-group that hold the rows of a KV head: the waves left over share the keys.
 template <typename KT, int HD>
 int launch(const dlk_attention_params& p, hipStream_t stream) {
-    const int rows = p.H / p.KV * p.L;
+    const int group = p.H / p.KV, rows = group * p.L;
     int wr = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
     // four row tiles that leave a CU with less than two work-groups: two, so that one's products run under another's
     // staging and softmax (4 x 510 causal positions, 8 / 2 heads of 32: 18.5 us at 256 work-groups, 15.2 at 512, 16.8 at
@@ -494,9 +513,9 @@ int launch(const dlk_attention_params& p, hipStream_t stream) {
     if (wr == 4 && static_cast<int64_t>((rows + 63) / 64) * p.splits * p.B * p.KV < 512) wr = 2;
     const dim3 grid(p.splits, (rows + 16 * wr - 1) / (16 * wr), p.B * p.KV);
     const dim3 threads(kThreads);
-    if (wr == 1) hipLaunchKernelGGL((attention_rows<KT, HD, 1>), grid, threads, 0, stream, p);
-    else if (wr == 2) hipLaunchKernelGGL((attention_rows<KT, HD, 2>), grid, threads, 0, stream, p);
-    else hipLaunchKernelGGL((attention_rows<KT, HD, 4>), grid, threads, 0, stream, p);
+    if (wr == 1) hipLaunchKernelGGL((attention_rows<KT, HD, 1>), grid, threads, 0, stream, p, group);
+    else if (wr == 2) hipLaunchKernelGGL((attention_rows<KT, HD, 2>), grid, threads, 0, stream, p, group);
+    else hipLaunchKernelGGL((attention_rows<KT, HD, 4>), grid, threads, 0, stream, p, group);
     const int status = static_cast<int>(hipGetLastError());
     if (status != 0 || p.splits == 1 || p.partials_only) return status;
     return launch_combine<HD, true>(p, stream);
