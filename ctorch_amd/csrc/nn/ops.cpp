@@ -129,7 +129,8 @@ void attention_split(Index batch, Index heads, Index kv_heads, Index head_dim, b
     // every CU has a work-group.  Measured on MI355X at 4 sequences x 7 positions over 1508 keys (32 such groups), us a
     // layer with its merge: 8 splits 16.3, 12 17.2, 24 (one tile each) 17.4; with 256 groups already (4 x 510 byte
     // positions) 3 splits took 58 against 19.
-    const Index groups = (heads / kv_heads * length + 63) / 64 * batch * kv_heads;
+    // (An empty chunk or batch has no work-group; its launch is refused later.)
+    const Index groups = std::max<Index>(1, (heads / kv_heads * length + 63) / 64 * batch * kv_heads);
     const Index wanted = std::max<Index>(1, 256 / groups);
     const Index tiles = std::max<Index>(1, (source + tile - 1) / tile);
     const Index per = std::max<Index>(2, (tiles + wanted - 1) / wanted);

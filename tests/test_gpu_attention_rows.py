@@ -109,3 +109,25 @@ def test_causal_chunks_over_a_prefix_match_the_oracle(batch, prefix, length, hea
     bound = 1e-4 if kv_dtype is None else 2e-2
     for part in (ids[:, :prefix], ids[:, prefix:]):
         assert rel_err(gpu.logits(part, gc), ref.logits(part, rc)[:, -1]) <= bound
+
+
+@pytest.mark.parametrize("batch,length", [(2, 0), (0, 3), (0, 20)])
+@pytest.mark.parametrize("heads,kv,hd", [(8, 2, 32), (4, 2, 64), (4, 2, 8)])
+def test_empty_queries_and_chunks_are_refused_and_leave_the_cache(batch, length, heads, kv, hd):
+    say(f"case: empty attention, {batch} x {length}, heads {heads}/{kv} of {hd}")
+    zeros = lambda *shape: ct.Tensor.from_numpy(np.zeros(shape, np.float32), ct.F32, GPU)
+    q, k = zeros(batch, heads, length, hd), zeros(batch, kv, 70, hd)
+    with pytest.raises(ct.DLError):
+        ct.grouped_query_attention(q, k, k, None)
+    empty = zeros(batch, length, heads * hd)
+    decoder = ct.transformer_decoder(1, heads * hd, heads, kv, 64, 32, ct.F32, GPU, 10000.0)
+    cache = ct.DecoderCache(decoder)
+    with pytest.raises(ct.DLError):
+        ct.decode(decoder, empty, cache)
+    assert cache.length == 0
+    if batch:  # the next chunk of that batch goes on as if the empty one had not been there
+        assert ct.decode(decoder, zeros(batch, 3, heads * hd), cache).shape == (batch, 3, heads * hd)
+        assert cache.length == 3
+        with pytest.raises(ct.DLError):
+            ct.decode(decoder, empty, cache)
+        assert cache.length == 3
