@@ -108,10 +108,10 @@ void* take_block(GpuContext& context, std::size_t& bytes) {
     if (!data) {
         int status = dlh_malloc_async(&data, bytes, context.stream);
         if (status != 0 && !captured && cache.held > 0) { // short of memory: the held blocks go back first
-            (void)dlh_last_launch_error();
             shrink(context, 0, 0);
             status = dlh_malloc_async(&data, bytes, context.stream);
         }
+        if (status != 0) (void)dlh_last_launch_error(); // the next launch must not report it again
         hip_check(status, "allocate");
     }
     cache.live += bytes;

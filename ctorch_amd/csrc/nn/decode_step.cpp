@@ -55,6 +55,17 @@ void DecodeWorkspace::attach_workspace(dlk_gemv_params& p, Device device) {
     p.split_capacity = split.numel();
 }
 
+void DecodeWorkspace::attach_workspace_if_room(dlk_gemv_params& p, Device device) {
+    if (static_cast<int64_t>(p.M) * p.K > (int64_t(1) << 30)) return;
+    dlk_gemv_params attached = p;
+    try {
+        attach_workspace(attached, device);
+    } catch (const std::runtime_error&) {
+        return;
+    }
+    p = attached;
+}
+
 const void* DecodeWorkspace::tiles_of(const Tensor& w0, const Tensor* w1, dlh_stream stream) {
     if (!pack_weights || w0.dtype() != DType::bf16 || w0.ndim() != 2 || !w0.is_contiguous()) return nullptr;
     const Index rows = w0.size(0), K = w0.size(1);

@@ -27,6 +27,10 @@ struct DecodeWorkspace {
     /// Points `p` at the staging workspace when its shape takes the tiled prefill path and at the split
     /// workspace when its launch would split the keys (both grown as needed).
     void attach_workspace(dlk_gemv_params& p, Device device);
+    /// The same for a projection called by itself, which must go on where only its own tensors fit the device: none over
+    /// more than 4 GiB of f32 rows (the staged copy is as large), and none where the allocation fails.  The launch
+    /// then takes 64 rows at a time.
+    void attach_workspace_if_room(dlk_gemv_params& p, Device device);
     void ensure(const nn::TransformerDecoderLayer& layer, Index rows, Index heads_total, Index hidden_features,
                 int splits, Device device);
 

@@ -43,9 +43,11 @@ Tensor SwiGLU::forward(const Tensor& input) {
     p.w_bf16 = gb;
     p.y = static_cast<float*>(mutable_data(act));
     p.ldy = F;
-    DecodeWorkspace ws;
-    ws.attach_workspace(p, input.device());
-    hip_check(dlk_gemv(&p, context.stream), "SwiGLU gate/up");
+    {
+        DecodeWorkspace ws;
+        ws.attach_workspace_if_room(p, input.device());
+        hip_check(dlk_gemv(&p, context.stream), "SwiGLU gate/up");
+    }
     return linear(act, down_->weight(), down_->bias());
 }
 
@@ -250,11 +252,19 @@ Tensor GroupedQueryAttention::run(const Tensor& input, KVCache* cache) {
     adapter_hidden(query_adapter_.get(), lq, 0);
     adapter_hidden(value_adapter_.get(), lv, 2);
     if (d % (qb ? 8 : 4) != 0) throw std::invalid_argument("attention width must be a multiple of 8");
-    DecodeWorkspace ws;
-    ws.attach_workspace(p, input.device());
+    dlk_attention_params a{};
+    attention_split(B, heads_, kv_heads_, hd, p.cache_bf16 != 0, L, offset + L, true, a.splits, a.chunk);
+    Tensor po, pml;
+    if (a.splits > 1) {
+        po = empty_tensor({B * heads_ * L, a.splits, hd}, DType::f32, input.device());
+        pml = empty_tensor({B * heads_ * L, a.splits, 2}, DType::f32, input.device());
+        a.partial_o = static_cast<float*>(mutable_data(po));
+        a.partial_ml = static_cast<float*>(mutable_data(pml));
+    }
+    DecodeWorkspace ws; // after the tensors that the call cannot do without
+    ws.attach_workspace_if_room(p, input.device());
     hip_check(dlk_gemv(&p, context.stream), "attention QKV");
 
-    dlk_attention_params a{};
     a.q = q.data<float>();
     a.ldq = heads_ * hd;
     a.k = target.key_data();
@@ -269,14 +279,6 @@ Tensor GroupedQueryAttention::run(const Tensor& input, KVCache* cache) {
     a.causal = 1;
     a.out = static_cast<float*>(mutable_data(attended));
     a.ldo = d;
-    attention_split(B, heads_, kv_heads_, hd, a.kv_bf16 != 0, L, offset + L, true, a.splits, a.chunk);
-    Tensor po, pml;
-    if (a.splits > 1) {
-        po = empty_tensor({B * heads_ * L, a.splits, hd}, DType::f32, input.device());
-        pml = empty_tensor({B * heads_ * L, a.splits, 2}, DType::f32, input.device());
-        a.partial_o = static_cast<float*>(mutable_data(po));
-        a.partial_ml = static_cast<float*>(mutable_data(pml));
-    }
     hip_check(dlk_attention(&a, context.stream), "attention");
 
     dlk_gemv_params o = gemv_params(attended.data<float>(), rows, d, DLK_EPI_STORE);
@@ -288,7 +290,7 @@ Tensor GroupedQueryAttention::run(const Tensor& input, KVCache* cache) {
     o.ldy = d;
     o.bump_position = target.position_data();
     o.bump_count = L;
-    ws.attach_workspace(o, input.device());
+    ws.attach_workspace_if_room(o, input.device());
     hip_check(dlk_gemv(&o, context.stream), "attention output");
     target.advance(L);
     return out;

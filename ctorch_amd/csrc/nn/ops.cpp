@@ -68,18 +68,15 @@ void linear_into(const float* x, Index rows, Index k, const Tensor& weight, cons
     p.w_bf16 = wb;
     p.y = y;
     p.ldy = ldy;
-    // the workspace of the staged kernels (released to the pool in stream order), as large as the rows: past 4 GiB of
-    // rows the launches of 64 rows, which need none, keep a product that fits the card only without it
-    DecodeWorkspace ws;
-    if (rows * k <= (Index{1} << 30)) ws.attach_workspace(p, weight.device());
+    Tensor b;
     if (bias) {
-        const Tensor b = bias->is_contiguous() ? *bias : bias->contiguous();
+        b = bias->is_contiguous() ? *bias : bias->contiguous();
         if (b.dtype() != DType::f32 && b.dtype() != DType::bf16) throw std::invalid_argument("linear: bias dtype");
         p.bias = b.data<void>();
         p.bias_bf16 = b.dtype() == DType::bf16;
-        hip_check(dlk_gemv(&p, context.stream), "linear");
-        return;
     }
+    DecodeWorkspace ws; // released to the pool in stream order
+    ws.attach_workspace_if_room(p, weight.device());
     hip_check(dlk_gemv(&p, context.stream), "linear");
 }
 

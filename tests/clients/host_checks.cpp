@@ -1,14 +1,105 @@
-// Prints what the library's host side decides for a call, without a GPU: linked from the library's own objects, because
-// these functions are not part of its exported surface.  Run by tests/test_host_rules.py.
+// What the library's host side decides for a call, without a GPU: linked from the library's own objects (these functions
+// are not part of its exported surface), with host memory and a list of the launches in the place of the device.  Run by
+// tests/test_host_rules.py.
 //
 //   host_checks split BATCH HEADS KV_HEADS HEAD_DIM KV_BF16 LENGTH SOURCE CAUSAL    attention_split: splits, keys per split
-#include "nn/ops_internal.h"
+//   host_checks workspace ENTRY ROWS K BYTES    launches of linear, swiglu or attention over bf16 weights with BYTES of
+//                                               device memory left for their workspaces (-1: no limit)
+#include "dl/decoder.h"
+#include "dl/gpu.h"
+#include "dl/ops.h"
+#include "nn/decode_step.h"
 
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <stdexcept>
+#include <string>
 
 namespace {
+
+struct Device {
+    std::map<void*, size_t> blocks; // allocations alive
+    size_t used = 0, peak = 0, limit = SIZE_MAX, launches = 0;
+    int last_error = 0;
+} fake;
+
+} // namespace
+
+// ------------------------------------------------------------------------- the backend, on host memory
+extern "C" {
+
+const char* dlh_error_string(int code) { return code == hipErrorOutOfMemory ? "out of memory" : "error"; }
+int dlh_device_count(int* count) { return *count = 1, 0; }
+int dlh_set_device(int) { return 0; }
+int dlh_get_device(int* device) { return *device = 0, 0; }
+int dlh_device_properties_get(int, dlh_device_properties* out) { return std::memset(out, 0, sizeof(*out)), 0; }
+int dlh_stream_create(dlh_stream* stream) { return *stream = reinterpret_cast<dlh_stream>(&fake), 0; }
+int dlh_stream_destroy(dlh_stream) { return 0; }
+int dlh_stream_synchronize(dlh_stream) { return 0; }
+int dlh_pool_configure(int) { return 0; }
+int dlh_malloc_async(void** pointer, size_t bytes, dlh_stream) {
+    if (bytes > fake.limit - std::min(fake.limit, fake.used)) return fake.last_error = hipErrorOutOfMemory;
+    *pointer = std::aligned_alloc(256, (bytes + 255) / 256 * 256); // never touched where the case is large
+    fake.blocks[*pointer] = bytes;
+    fake.peak = std::max(fake.peak, fake.used += bytes);
+    return 0;
+}
+int dlh_free_async(void* pointer, dlh_stream) {
+    fake.used -= fake.blocks.at(pointer);
+    fake.blocks.erase(pointer);
+    std::free(pointer);
+    return 0;
+}
+int dlh_pool_stats(int, uint64_t* used, uint64_t* reserved, uint64_t* peak_used, uint64_t* peak_reserved, uint64_t* threshold) {
+    *used = *reserved = fake.used;
+    *peak_used = *peak_reserved = fake.peak;
+    return *threshold = UINT64_MAX, 0;
+}
+int dlh_pool_trim(int) { return 0; }
+int dlh_pool_set_threshold(int, uint64_t) { return 0; }
+int dlh_pool_reset_peaks(int) { return fake.peak = fake.used, 0; }
+int dlh_memcpy_async(void* to, const void* from, size_t bytes, int, dlh_stream) { return std::memcpy(to, from, bytes), 0; }
+int dlh_event_create(dlh_event*) { return 0; }
+int dlh_event_destroy(dlh_event) { return 0; }
+int dlh_event_record(dlh_event, dlh_stream) { return 0; }
+int dlh_event_synchronize(dlh_event) { return 0; }
+int dlh_event_elapsed(dlh_event, dlh_event, float* ms) { return *ms = 0, 0; }
+int dlh_capture_begin(dlh_stream) { return 0; }
+int dlh_stream_capturing(dlh_stream, int* capturing) { return *capturing = 0, 0; }
+int dlh_capture_end(dlh_stream, dlh_graph*) { return 0; }
+int dlh_graph_launch(dlh_graph, dlh_stream) { return 0; }
+int dlh_graph_destroy(dlh_graph) { return 0; }
+int dlh_last_launch_error(void) { return std::exchange(fake.last_error, 0); }
+
+// the runtime functions that the launch code calls: a launch counts, and reports an error that an earlier call left
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) {
+    fake.launches += 1;
+    return static_cast<hipError_t>(std::exchange(fake.last_error, 0));
+}
+static thread_local struct { dim3 grid, block; size_t lds; hipStream_t stream; } configured; // of a <<<>>> launch
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t stream) {
+    configured = {grid, block, lds, stream};
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* lds, hipStream_t* stream) {
+    *grid = configured.grid, *block = configured.block, *lds = configured.lds, *stream = configured.stream;
+    return hipSuccess;
+}
+hipError_t hipGetLastError(void) { return static_cast<hipError_t>(std::exchange(fake.last_error, 0)); }
+hipError_t hipGetDevice(int* device) { return *device = 0, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* value, hipDeviceAttribute_t, int) { return *value = 256, hipSuccess; }
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* blocks, const void*, int, size_t) { return *blocks = 4, hipSuccess; }
+
+} // extern "C"
+
+namespace {
+
+using dl::detail::empty_tensor;
 
 int split(char** arg) {
     int splits = 0, chunk = 0;
@@ -18,10 +109,44 @@ int split(char** arg) {
     return 0;
 }
 
+int workspace(char** arg) {
+    const std::string entry = arg[0];
+    const dl::Index rows = std::atoll(arg[1]), k = std::atoll(arg[2]), left = std::atoll(arg[3]);
+    const dl::Device gpu = dl::Device::gpu(0);
+    const dl::TensorOptions options{.dtype = dl::DType::bf16, .device = gpu};
+    const dl::Index n = 512;
+    const dl::Tensor x = empty_tensor({1, rows, k}, dl::DType::f32, gpu), w = empty_tensor({n, k}, dl::DType::bf16, gpu);
+    dl::nn::SwiGLU swiglu(k, n, false, options);
+    dl::nn::GroupedQueryAttention attention(k, k / 128, k / 256, entry == "attention" ? rows : 1, options);
+    auto call = [&] {
+        if (entry == "linear") (void)dl::linear(x, w);
+        else if (entry == "swiglu") (void)swiglu.forward(x);
+        else if (entry == "attention") (void)attention.forward(x);
+        else throw std::invalid_argument("entry");
+    };
+    dl::gpu::set_memory_release_threshold(0); // no freed blocks held
+    const size_t before = fake.used;
+    dl::Index own = 0; // bytes of the tensors that the call needs whatever it launches
+    if (entry == "linear") own = rows * n * 4;
+    if (entry == "swiglu") own = rows * (n + k) * 4;
+    if (entry == "attention") own = rows * 3 * k * 4 + 2 * rows * (k / 2) * 4 + (1 << 12); // q, attended, out; the local cache
+    if (left >= 0) fake.limit = before + static_cast<size_t>(own + left);
+    fake.launches = 0;
+    call();
+    std::printf("%zu\n", fake.launches);
+    return 0;
+}
+
 } // namespace
 
 int main(int argc, char** argv) {
-    if (argc == 10 && std::strcmp(argv[1], "split") == 0) return split(argv + 2);
-    std::fprintf(stderr, "usage: host_checks split BATCH HEADS KV_HEADS HEAD_DIM KV_BF16 LENGTH SOURCE CAUSAL\n");
+    try {
+        if (argc == 10 && std::strcmp(argv[1], "split") == 0) return split(argv + 2);
+        if (argc == 6 && std::strcmp(argv[1], "workspace") == 0) return workspace(argv + 2);
+    } catch (const std::exception& error) {
+        std::fprintf(stderr, "%s\n", error.what());
+        return 1;
+    }
+    std::fprintf(stderr, "see the head of host_checks.cpp\n");
     return 2;
 }

@@ -29,3 +29,19 @@ def test_an_empty_chunk_or_batch_has_a_split(batch, length, head_dim, source, ca
     for kv_bf16 in (False, True):
         splits, chunk = split(batch, 8, 2, head_dim, kv_bf16, length, source, causal)
         assert splits >= 0 and chunk >= 0
+
+
+@pytest.mark.parametrize("entry,staged,by_64_rows", [("linear", 3, 5), ("swiglu", 6, 10), ("attention", 8, 12)])
+def test_a_call_that_fits_only_without_its_workspace_goes_on_without(entry, staged, by_64_rows):
+    """300 rows of 512: a staged projection is three launches (rows, product, key slices), one without it five of 64
+    rows; the attention module adds the fill of its cache's length and the attention itself."""
+    assert int(checks("workspace", entry, 300, 512, -1)) == staged
+    for left in (0, 1 << 16, 300 * 512 * 4):
+        assert int(checks("workspace", entry, 300, 512, left)) == by_64_rows
+
+
+@pytest.mark.parametrize("entry", ["linear", "swiglu", "attention"])
+def test_no_staged_copy_past_4_gib_of_rows(entry):
+    # the buffers are reserved, not touched
+    few, many = (int(checks("workspace", entry, rows, 4096, -1)) for rows in (1 << 18, (1 << 18) + 1))
+    assert few < 20 and many >= (1 << 18) // 64
