@@ -1,12 +1,12 @@
-// Projection over several activation rows with f32 weights, with the epilogues of the GEMV (see dlk_gemv_params in
-// kernels.h), on the f32 matrix cores.
+// Projection over several activation rows on the f32 matrix cores, with the epilogues of the GEMV (see dlk_gemv_params in
+// kernels.h): f32 weights, and bf16 weights of the shapes that no bf16 matrix-core kernel takes with whole f32 activations.
 //
 // One v_mfma_f32_16x16x4_f32 computes D[16 weight rows][16 activation rows] += W[16][4] * X[16][4]^T in f32: lane l
 // supplies one weight of row l%16 and one activation of row l%16 at k slot l/16, and receives D[rows 4(l/16) .. +4]
 // [l%16].  The k slots of four products are dealt so that a lane's operands are four consecutive k (k slot l/16 of
 // product j is k 4(l/16) + j), so the fragments of 16 k are one 16-byte LDS read per tile.
 //
-// Work-group: four waves, WN x WM, each owning TN x TM tiles of 16 x 16.  Both operands are staged in LDS as they are,
+// Work-group: four waves, WN x WM, each owning TN x TM tiles of 16 x 16.  Both operands are staged in LDS as f32,
 // 32 k at a time, double buffered, the next chunk's loads in flight (in registers) while one is used.  A product rounds
 // its sum after every k, so one accumulator over a long K would lose what the GEMV's 64 short sums keep (K = 4096:
 // 1.1e-6 against 64-bit results, the GEMV 1.1e-7): each 16 k start from zero and are added up in f64 (the vector ALU
@@ -27,6 +27,7 @@ namespace dlk::gemm32 {
 
 using gemm::f32x4;
 using gemm::kTile;
+using gemv::u32x4;
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 constexpr int kThreads = 256;
 constexpr int kWaveChunk = 32;           // k per wave and staged chunk
@@ -51,11 +52,21 @@ __host__ __device__ inline int col_blocks(const dlk_gemv_params& p, int rows) {
     return (tiles_of(p) + per - 1) / per;
 }
 
-/// Whether this kernel takes the launch (host side): from the third launch that the GEMV would need, which takes one
-/// to four activation rows at a time (K > 3072: one) and streams the weights again for each.
+/// Whether this kernel takes the launch (host side; bf16 weights: one that the kernels which split the activations into
+/// two bf16 parts leave, see gemv.hip).
+/// f32 weights: from the third launch that the GEMV would need, which takes one to four activation rows at a time (K >
+/// 3072: one) and streams the weights again for each.
+/// bf16 weights: over 65 rows and more, any width, K in whole pairs of k steps.  The activations stay whole as in the
+/// GEMV (7.8e-8 against 64-bit results; the GEMV 0.7e-7 to 1.0e-7, two bf16 parts 2.5e-6), and the weights become f32 while
+/// they are staged.  Measured on MI355X against the GEMV, us: 65 x 320 -> 640 97 -> 8.5, 100 x 4096 -> 8191 1113 -> 122,
+/// 333 x 2048 -> 32001 3538 -> 532, 2000 x 4096 -> 15999 40617 -> 2612 (gemm_mid's two parts: 12, 55, 115, 553).
+/// Fewer rows, other K and several segments that are no multiple of 16 were not measured and stay with the GEMV.
 inline bool eligible(const dlk_gemv_params& p) {
-    if (p.w_bf16 || p.epilogue == DLK_EPI_LOGITS || p.K % 4 != 0 || p.ldx % 4 != 0) return false;
-    if (p.M <= 2 * gemv::plan_of(p.K, false, p.epilogue).mt_max) return false;
+    if (p.epilogue == DLK_EPI_LOGITS || p.K % (p.w_bf16 ? 64 : 4) != 0 || p.ldx % 4 != 0) return false;
+    if (p.M <= (p.w_bf16 ? gemm::kMaxRows : 2 * gemv::plan_of(p.K, false, p.epilogue).mt_max)) return false;
+    if (p.w_bf16)
+        for (int s = 0; s < p.nseg; ++s)
+            if (p.nseg == 1 ? p.seg_rows[s] < kTile : p.seg_rows[s] % kTile != 0) return false;
     auto aligned = [](const void* q, uintptr_t bytes) { return reinterpret_cast<uintptr_t>(q) % bytes == 0; };
     if (!aligned(p.x, 16)) return false;
     for (int s = 0; s < p.nseg; ++s)
@@ -90,17 +101,18 @@ inline int shape_of(const dlk_gemv_params& p) {
 // A tile of 16 weight rows: its segment, first row, rows of the segment.
 struct Tile {
     int seg, n0, rows;
-    const float* base;
+    const void* base;
 };
 __device__ __forceinline__ Tile locate(const dlk_gemv_params& p, int tile) {
     const int t0 = segment_tiles(p.seg_rows[0]), t1 = p.nseg > 1 ? segment_tiles(p.seg_rows[1]) : 0;
-    if (tile < t0 || p.nseg == 1) return {0, tile * kTile, p.seg_rows[0], static_cast<const float*>(p.w[0])};
+    if (tile < t0 || p.nseg == 1) return {0, tile * kTile, p.seg_rows[0], p.w[0]};
     if (tile < t0 + t1 || p.nseg == 2)
-        return {1, (tile - t0) * kTile, p.seg_rows[1], static_cast<const float*>(p.w[1])};
-    return {2, (tile - t0 - t1) * kTile, p.seg_rows[2], static_cast<const float*>(p.w[2])};
+        return {1, (tile - t0) * kTile, p.seg_rows[1], p.w[1]};
+    return {2, (tile - t0 - t1) * kTile, p.seg_rows[2], p.w[2]};
 }
 
-template <int EPI, bool NORM, int WN, int WM, int WK, int TN, int TM>
+// WT: float, or uint16_t for bf16 weights.
+template <typename WT, int EPI, bool NORM, int WN, int WM, int WK, int TN, int TM>
 __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
     constexpr bool SWIGLU = EPI == DLK_EPI_SWIGLU;
     constexpr int BN = kTile * WN * TN, BM = kTile * WM * TM;
@@ -109,9 +121,11 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
     constexpr int kStride = kChunk + 8;
     constexpr int kPieces = kChunk / 4;              // 16-byte pieces per staged row
     constexpr int kRowsPerPass = kThreads / kPieces;
-    constexpr int WLOADS = BN / kRowsPerPass, XLOADS = (BM + kRowsPerPass - 1) / kRowsPerPass;
+    constexpr int VALUES = 16 / sizeof(WT);          // weights per 16-byte piece
+    constexpr int kWeightPieces = kChunk / VALUES, kWeightRowsPerPass = kThreads / kWeightPieces;
+    constexpr int WLOADS = BN / kWeightRowsPerPass, XLOADS = (BM + kRowsPerPass - 1) / kRowsPerPass;
     constexpr int FT = BN / kTile / 2; // SwiGLU: gate tiles of a work-group
-    static_assert(WN * WM * WK * kWave == kThreads && BN % kRowsPerPass == 0 && (!SWIGLU || TN % 2 == 0), "shape");
+    static_assert(WN * WM * WK * kWave == kThreads && BN % kWeightRowsPerPass == 0 && (!SWIGLU || TN % 2 == 0), "shape");
     __shared__ __attribute__((aligned(16))) float ws[2][BN][kStride];
     __shared__ __attribute__((aligned(16))) float xs[2][BM][kStride];
 
@@ -131,18 +145,18 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
 
     // staging: thread t takes one 16-byte piece of rows t / kPieces, + kRowsPerPass, ...; rows past the end repeat the
     // last
-    const int piece = t % kPieces, row = t / kPieces;
-    const float* wp[WLOADS];
+    const int piece = t % kPieces, row = t / kPieces, weight_piece = t % kWeightPieces, weight_row = t / kWeightPieces;
+    const WT* wp[WLOADS];
 #pragma unroll
     for (int i = 0; i < WLOADS; ++i) {
-        const int b = row + i * kRowsPerPass; // weight row of the work-group
+        const int b = weight_row + i * kWeightRowsPerPass; // weight row of the work-group
         if constexpr (SWIGLU) {
             const bool up = b >= FT * kTile;
             const int n = min(tile0 * kTile + (up ? b - FT * kTile : b), p.seg_rows[0] - 1);
-            wp[i] = static_cast<const float*>(up ? p.w[1] : p.w[0]) + static_cast<int64_t>(n) * K;
+            wp[i] = static_cast<const WT*>(up ? p.w[1] : p.w[0]) + static_cast<int64_t>(n) * K;
         } else {
             const Tile tile = locate(p, min(tile0 + b / kTile, tiles - 1));
-            wp[i] = tile.base + static_cast<int64_t>(min(tile.n0 + b % kTile, tile.rows - 1)) * K;
+            wp[i] = static_cast<const WT*>(tile.base) + static_cast<int64_t>(min(tile.n0 + b % kTile, tile.rows - 1)) * K;
         }
     }
     const float* xp[XLOADS];
@@ -151,7 +165,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
         xp[i] = p.x + static_cast<int64_t>(min(m0 + row + i * kRowsPerPass, p.M - 1)) * p.ldx;
     const bool affine = NORM && p.apply_norm && p.norm_weight;
 
-    f32x4 wr[WLOADS], xr[XLOADS], g = {1.f, 1.f, 1.f, 1.f};
+    u32x4 wr[WLOADS];
+    f32x4 xr[XLOADS], g = {1.f, 1.f, 1.f, 1.f};
     auto load = [&](int chunk) {
         const int k = min(chunk * kChunk + 4 * piece, K - 4);
 #pragma unroll
@@ -165,7 +180,8 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
             }
         }
 #pragma unroll
-        for (int i = 0; i < WLOADS; ++i) wr[i] = *reinterpret_cast<const f32x4*>(wp[i] + k);
+        for (int i = 0; i < WLOADS; ++i)
+            wr[i] = *reinterpret_cast<const u32x4*>(wp[i] + min(chunk * kChunk + VALUES * weight_piece, K - VALUES));
     };
     float squares[XLOADS] = {};
     auto stage = [&](int chunk, int buf) {
@@ -182,8 +198,16 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
                 *reinterpret_cast<f32x4*>(&xs[buf][row + i * kRowsPerPass][4 * piece]) = v;
         }
 #pragma unroll
-        for (int i = 0; i < WLOADS; ++i)
-            *reinterpret_cast<f32x4*>(&ws[buf][row + i * kRowsPerPass][4 * piece]) = live ? wr[i] : zero;
+        for (int i = 0; i < WLOADS; ++i) {
+            float* to = &ws[buf][weight_row + i * kWeightRowsPerPass][VALUES * weight_piece];
+            const u32x4 w = chunk * kChunk + VALUES * weight_piece < K ? wr[i] : u32x4{0u, 0u, 0u, 0u};
+            if constexpr (VALUES == 4) {
+                *reinterpret_cast<u32x4*>(to) = w;
+            } else {
+                *reinterpret_cast<f32x4*>(to) = f32x4{bf16_lo(w.x), bf16_hi(w.x), bf16_lo(w.y), bf16_hi(w.y)};
+                *reinterpret_cast<f32x4*>(to + 4) = f32x4{bf16_lo(w.z), bf16_hi(w.z), bf16_lo(w.w), bf16_hi(w.w)};
+            }
+        }
     };
 
     // a wave's weight tiles: generic TN consecutive ones; SwiGLU TN / 2 gate tiles, then the up tiles of the same
@@ -333,13 +357,16 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
                     const float* hidden = tm.seg == 0 ? p.lora_hidden[0] : tm.seg == 2 ? p.lora_hidden[2] : nullptr;
                     if (hidden) {
                         // unmerged LoRA: + scale * up[n, :] . hidden[m, :] (rows past the segment repeat its last)
-                        const float* up = static_cast<const float*>(tm.seg == 0 ? p.lora_up[0] : p.lora_up[2]);
+                        const WT* up = static_cast<const WT*>(tm.seg == 0 ? p.lora_up[0] : p.lora_up[2]);
                         const float* h = hidden + mg * gemv::lora_stride(p);
                         float d[4] = {0.f, 0.f, 0.f, 0.f};
                         for (int k = 0; k < p.lora_rank; ++k) {
 #pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                d[e] += up[static_cast<int64_t>(min(n + e, tm.rows - 1)) * p.lora_rank + k] * h[k];
+                            for (int e = 0; e < 4; ++e) {
+                                const WT value = up[static_cast<int64_t>(min(n + e, tm.rows - 1)) * p.lora_rank + k];
+                                if constexpr (sizeof(WT) == 4) d[e] += value * h[k];
+                                else d[e] += bf16_to_f32(value) * h[k];
+                            }
                         }
 #pragma unroll
                         for (int e = 0; e < 4; ++e) v[e] += d[e] * p.lora_scale;
@@ -377,25 +404,30 @@ __global__ __launch_bounds__(kThreads) void gemm_f32(const dlk_gemv_params p) {
     }
 }
 
-template <int EPI, bool NORM>
+template <typename WT, int EPI, bool NORM>
 const void* shape_kernel(int shape) {
     switch (shape) {
-    case k128x128: return reinterpret_cast<const void*>(&gemm_f32<EPI, NORM, 2, 2, 1, 4, 4>);
-    case k64x64: return reinterpret_cast<const void*>(&gemm_f32<EPI, NORM, 2, 2, 1, 2, 2>);
-    case k64x32: return reinterpret_cast<const void*>(&gemm_f32<EPI, NORM, 2, 2, 1, 2, 1>);
-    case k32x16: return reinterpret_cast<const void*>(&gemm_f32<EPI, NORM, 1, 1, 4, 2, 1>);
+    case k128x128: return reinterpret_cast<const void*>(&gemm_f32<WT, EPI, NORM, 2, 2, 1, 4, 4>);
+    case k64x64: return reinterpret_cast<const void*>(&gemm_f32<WT, EPI, NORM, 2, 2, 1, 2, 2>);
+    case k64x32: return reinterpret_cast<const void*>(&gemm_f32<WT, EPI, NORM, 2, 2, 1, 2, 1>);
+    case k32x16: return reinterpret_cast<const void*>(&gemm_f32<WT, EPI, NORM, 1, 1, 4, 2, 1>);
     default: return nullptr;
     }
+}
+
+template <int EPI, bool NORM>
+const void* weight_kernel(const dlk_gemv_params& p, int shape) {
+    return p.w_bf16 ? shape_kernel<uint16_t, EPI, NORM>(shape) : shape_kernel<float, EPI, NORM>(shape);
 }
 
 /// The kernel of a launch for a work-group shape; null if none.
 template <int EPI>
 const void* resolve(const dlk_gemv_params& p, int shape) {
     if (gemv::norm_variant(EPI, p.apply_norm != 0)) {
-        if constexpr (EPI != DLK_EPI_RESIDUAL) return shape_kernel<EPI, true>(shape);
+        if constexpr (EPI != DLK_EPI_RESIDUAL) return weight_kernel<EPI, true>(p, shape);
         return nullptr;
     }
-    if constexpr (EPI == DLK_EPI_STORE || EPI == DLK_EPI_RESIDUAL) return shape_kernel<EPI, false>(shape);
+    if constexpr (EPI == DLK_EPI_STORE || EPI == DLK_EPI_RESIDUAL) return weight_kernel<EPI, false>(p, shape);
     return nullptr;
 }
 

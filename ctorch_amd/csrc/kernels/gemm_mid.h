@@ -18,9 +18,9 @@
 // pair takes 0.9 us against 0.45 us of products.  Deeper rings with a stream per wave (four pairs of weights and three of
 // activations, or five and two) and fragments read a pair ahead of their products changed that by -10 to +2%, so neither
 // is there.  The smallest launches are round trips (7 us for a single pair).  Measured on MI355X (the launches that it
-// replaces: gemm_rows 64 rows at a time with its reduces, gemm_tiles with most CUs idle, the GEMV for odd widths), us
-// with the split pass and the reduce: 200 rows 2048 -> 3072 55.7 -> 26.1, 2048 -> 11264 107 -> 37.6, 5632 -> 2048 67.4 -> 28.2;
-// 1013 rows 4096 -> 4096 155 -> 71, 14336 -> 4096 496 -> 222; 100 rows 4096 -> 8191 1170 -> 57.
+// replaces: gemm_rows 64 rows at a time with its reduces, gemm_tiles with most CUs idle), us with the split pass and the
+// reduce: 200 rows 2048 -> 3072 55.7 -> 26.1, 2048 -> 11264 107 -> 37.6, 5632 -> 2048 67.4 -> 28.2;
+// 1013 rows 4096 -> 4096 155 -> 71, 14336 -> 4096 496 -> 222.
 #pragma once
 
 #include "kernels/gemm_tiles.h"
@@ -46,10 +46,9 @@ constexpr int kDma = 6;                      // DMA instructions per wave and pa
 static_assert(kStages * (kWeightBytes + kActBytes) <= 160 * 1024 &&
                   (2 * kBM * kOutStride + kBM) * 4 <= kStages * (kWeightBytes + kActBytes), "LDS");
 
-/// 16-row weight tiles (a lone segment's last tile may overlap the one before it; SwiGLU: gate tiles).
+/// 16-row weight tiles (SwiGLU: gate tiles).
 __host__ __device__ inline int tiles_of(const dlk_gemv_params& p) {
-    if (p.epilogue == DLK_EPI_SWIGLU) return p.seg_rows[0] / kTile;
-    return p.nseg == 1 ? (p.seg_rows[0] + kTile - 1) / kTile : gemm::tiles_of(p);
+    return p.epilogue == DLK_EPI_SWIGLU ? p.seg_rows[0] / kTile : gemm::tiles_of(p);
 }
 __host__ __device__ inline int col_blocks(const dlk_gemv_params& p) {
     const int per = kBN / kTile / (p.epilogue == DLK_EPI_SWIGLU ? 2 : 1);
@@ -61,8 +60,6 @@ __host__ __device__ inline int row_blocks(const dlk_gemv_params& p) { return (p.
 /// MI355X at 200 rows (us, with the reduce): at most 256 / 192 / 128 work-groups, 2048 -> 2048 and 5632 -> 2048 on average
 /// 22.4 / 23.6 / 25.8, QKV 2048 -> 3072 23.1 / 24.2 / 27.3; gate/up of 128 rows (88 work-groups) 34 in one slice, 29 in two.
 inline int splits_of(const dlk_gemv_params& p) {
-    for (int s = 0; s < p.nseg; ++s)
-        if (p.seg_rows[s] % kTile != 0) return 1;
     const int blocks = col_blocks(p) * row_blocks(p);
     return std::max(1, std::min({256 / blocks, gemm::kMaxSplits, p.K / 64 / 4}));
 }
@@ -71,8 +68,7 @@ inline int64_t split_floats(const dlk_gemv_params& p) { // the layout that gemm_
     return splits <= 1 ? 0 : static_cast<int64_t>(splits) * p.M * (gemm::tiles_of(p) * kTile + 1);
 }
 
-/// Whether this kernel takes the shape (host side): the conditions of the tiled projection without its row count, and
-/// any number of weight rows in a lone segment.
+/// Whether this kernel takes the shape (host side): the conditions of the tiled projection without its row count.
 inline bool shape_eligible(const dlk_gemv_params& p) {
     auto aligned = [](const void* at, uintptr_t bytes) { return reinterpret_cast<uintptr_t>(at) % bytes == 0; };
     if (!p.w_bf16 || p.epilogue == DLK_EPI_LOGITS || p.K % 64 != 0 || p.M < kMinRows) return false;
@@ -80,7 +76,7 @@ inline bool shape_eligible(const dlk_gemv_params& p) {
     if (p.apply_norm && p.norm_weight && !aligned(p.norm_weight, 16)) return false;
     for (int s = 0; s < p.nseg; ++s) {
         if (!aligned(p.w[s], 16)) return false;
-        if (p.nseg == 1 ? p.seg_rows[s] < kTile : p.seg_rows[s] % kTile != 0) return false;
+        if (p.seg_rows[s] % kTile != 0) return false;
     }
     if (p.epilogue == DLK_EPI_SWIGLU && (p.ldy % 4 != 0 || !aligned(p.y, 16))) return false;
     // four head-dim entries of one head per store
@@ -90,24 +86,19 @@ inline bool shape_eligible(const dlk_gemv_params& p) {
     return static_cast<int64_t>(kTile) * p.K * 2 < (int64_t(1) << 31); // 32-bit DMA lane offsets
 }
 
-// Weight rows of work-group tile T as a row base: the tile's first row, pulled back where the segment ends inside it.
+// Weight rows of work-group tile T: its segment and first row.
 struct Tile {
-    int seg, n0, skip; // skip: leading rows of the tile that the one before it covers
+    int seg, n0;
     const uint16_t* base;
 };
 template <bool SWIGLU>
 __device__ __forceinline__ Tile locate(const dlk_gemv_params& p, int n_blk, int T, int tiles) {
     if constexpr (SWIGLU) {
         const int f = kTile * min(n_blk * (kBN / kTile / 2) + T % (kBN / kTile / 2), tiles - 1);
-        return {0, f, 0, static_cast<const uint16_t*>(p.w[T < kBN / kTile / 2 ? 0 : 1])};
+        return {0, f, static_cast<const uint16_t*>(p.w[T < kBN / kTile / 2 ? 0 : 1])};
     } else {
-        const int tile = min(n_blk * (kBN / kTile) + T, tiles - 1);
-        if (p.nseg == 1) {
-            const int n0 = min(tile * kTile, p.seg_rows[0] - kTile);
-            return {0, n0, tile * kTile - n0, static_cast<const uint16_t*>(p.w[0])};
-        }
-        const gemm::TileMap tm = gemm::locate<false>(p, tile);
-        return {tm.seg, tm.n0, 0, tm.base0};
+        const gemm::TileMap tm = gemm::locate<false>(p, min(n_blk * (kBN / kTile) + T, tiles - 1));
+        return {tm.seg, tm.n0, tm.base0};
     }
 }
 
@@ -216,7 +207,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mid(const dlk_gemv_params p)
     const int n = tm.n0 + col % kTile; // first weight row (feature) of the outputs
     const int64_t width = static_cast<int64_t>(gemm::tiles_of(p)) * kTile; // of a partial row
     const bool finish = splits == 1;
-    const bool vec = p.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0 && tm.skip == 0 &&
+    const bool vec = p.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(p.y) % 16 == 0 &&
                      (EPI != DLK_EPI_RESIDUAL || (p.ldres % 4 == 0 && reinterpret_cast<uintptr_t>(p.residual) % 16 == 0));
     f32x4 residual[PASSES];
     if constexpr (EPI == DLK_EPI_RESIDUAL) {
@@ -339,8 +330,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mid(const dlk_gemv_params p)
             } else {
                 const float* res = EPI == DLK_EPI_RESIDUAL ? p.residual + static_cast<int64_t>(m) * p.ldres + n : nullptr;
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (col % kTile + e >= tm.skip) y[e] = EPI == DLK_EPI_RESIDUAL ? v[e] + res[e] : v[e];
+                for (int e = 0; e < 4; ++e) y[e] = EPI == DLK_EPI_RESIDUAL ? v[e] + res[e] : v[e];
             }
         }
     }

@@ -570,8 +570,6 @@ constexpr int kNarrowBatch = 4; // k steps per batch of loads (two batches in fl
 
 /// Whether a staged launch takes gemm_narrow (host side).
 inline bool narrow_eligible(const dlk_gemv_params& p) {
-    for (int s = 0; s < p.nseg; ++s)
-        if (p.seg_rows[s] % gemm::kTile != 0) return false;
     return p.epilogue == DLK_EPI_STORE && !p.bias && gemm::tiles_of(p) <= 2 && p.ldy % 4 == 0 &&
            reinterpret_cast<uintptr_t>(p.y) % 16 == 0;
 }

@@ -1,7 +1,8 @@
 // Host dispatch of the projections: the GEMV (gemv_impl.h) for one or two activation rows (or shapes the matrix
 // cores do not take), the matrix-core kernel (gemm_rows.h) for a batch of decode rows, and the tiled matrix-core
 // kernels for prompts and prefill chunks (gemm_tiles.h, gemm_mid.h where its tiles would not fill the device), and with
-// f32 weights the f32 matrix-core kernel (gemm_f32.h); all instantiated per epilogue in gemv_*.hip.
+// f32 weights, or over many rows of a shape that the others leave, the f32 matrix-core kernel (gemm_f32.h); all
+// instantiated per epilogue in gemv_*.hip.
 //
 // The grid is persistent: one wave per row group, capped at the number of waves the chosen kernel keeps
 // resident on the device (its occupancy times the CU count), so every wave streams from the start and none
@@ -61,8 +62,12 @@ Kernel resolve_tiles(const dlk_gemv_params& p) {
     }
 }
 
-/// A shape that one of the staged kernels (gemm_tiles, gemm_mid, gemm_narrow) takes.
-bool staged_shape(const dlk_gemv_params& p) { return dlk::tiles::shape_eligible(p) || dlk::mid::shape_eligible(p); }
+/// A shape that one of the staged kernels (gemm_tiles, gemm_mid, gemm_narrow) takes.  They split the activations into two
+/// bf16 parts (2.5e-6 of the result against 64 bits).  gemm_rows does the same, so the shapes it takes lose nothing by
+/// gemm_mid; the others would go to the GEMV, whose activations are whole (1e-7), and stay so (gemm_f32).
+bool staged_shape(const dlk_gemv_params& p) {
+    return dlk::tiles::shape_eligible(p) || (dlk::mid::shape_eligible(p) && dlk::gemm::eligible(p));
+}
 
 /// The staged kernels run when the shape suits one and the caller attached the staging workspace.
 bool staged(const dlk_gemv_params& p) {
@@ -81,8 +86,6 @@ bool use_mid(const dlk_gemv_params& p) {
     return rounds(static_cast<int64_t>(dlk::mid::col_blocks(p)) * dlk::mid::row_blocks(p)) * 63 <
            rounds(static_cast<int64_t>(dlk::tiles::col_blocks(p)) * dlk::tiles::row_blocks(p)) * 181;
 }
-
-Kernel resolve_reduce(const dlk_gemv_params& p);
 
 int launch_reduce(dlk_gemv_params& p, int splits, hipStream_t stream) {
     using namespace dlk::gemm;
@@ -228,7 +231,7 @@ int launch_gemm(const dlk_gemv_params& params, hipStream_t stream) {
     return 0;
 }
 
-// f32 weights over several rows: one launch over all rows.
+// Several rows on the f32 matrix cores: one launch over all rows.
 int launch_f32(const dlk_gemv_params& p, hipStream_t stream) {
     using namespace dlk::gemm32;
     const int shape = shape_of(p);

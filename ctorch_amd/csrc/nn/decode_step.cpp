@@ -56,7 +56,7 @@ void DecodeWorkspace::attach_workspace(dlk_gemv_params& p, Device device) {
 }
 
 void DecodeWorkspace::attach_workspace_if_room(dlk_gemv_params& p, Device device) {
-    if (static_cast<int64_t>(p.M) * p.K > (int64_t(1) << 30)) return;
+    if (!dlk_gemv_uses_rows(&p) || static_cast<int64_t>(p.M) * p.K > (int64_t(1) << 30)) return;
     dlk_gemv_params attached = p;
     try {
         attach_workspace(attached, device);

@@ -29,7 +29,8 @@ struct DecodeWorkspace {
     void attach_workspace(dlk_gemv_params& p, Device device);
     /// The same for a projection called by itself, which must go on where only its own tensors fit the device: none over
     /// more than 4 GiB of f32 rows (the staged copy is as large), and none where the allocation fails.  The launch
-    /// then takes 64 rows at a time.
+    /// then takes 64 rows at a time.  None either where those launches keep the activations in f32 (the widths and K that
+    /// gemm_rows does not take): the staged kernels split them into two bf16 parts.
     void attach_workspace_if_room(dlk_gemv_params& p, Device device);
     void ensure(const nn::TransformerDecoderLayer& layer, Index rows, Index heads_total, Index hidden_features,
                 int splits, Device device);
