@@ -89,10 +89,11 @@ void shrink(GpuContext& context, std::size_t bytes, std::size_t blocks) {
     }
 }
 
-// a block of at least `bytes`, which receives its size
-void* take_block(GpuContext& context, std::size_t& bytes) {
+// a block of at least `bytes`, which receives its size, and whether a capture recorded the allocation
+void* take_block(GpuContext& context, std::size_t& bytes, bool& captured) {
     auto& cache = context.cache;
-    const bool captured = capturing(context), direct = captured || bytes > BlockCache::kBlockMax;
+    captured = capturing(context);
+    const bool direct = captured || bytes > BlockCache::kBlockMax;
     std::lock_guard<std::mutex> lock(cache.mutex);
     void* data = nullptr;
     if (!direct) {
@@ -119,10 +120,11 @@ void* take_block(GpuContext& context, std::size_t& bytes) {
     return data;
 }
 
-void give_block(GpuContext& context, void* data, std::size_t bytes) {
+void give_block(GpuContext& context, void* data, std::size_t bytes, bool captured) {
     auto& cache = context.cache;
     int active = 0;
-    const bool direct = bytes > BlockCache::kBlockMax || dlh_stream_capturing(context.stream, &active) != 0 || active != 0;
+    const bool direct = captured || bytes > BlockCache::kBlockMax ||
+                        dlh_stream_capturing(context.stream, &active) != 0 || active != 0;
     std::lock_guard<std::mutex> lock(cache.mutex);
     cache.live -= bytes;
     bool kept = false;
@@ -149,7 +151,7 @@ Storage::~Storage() {
         std::free(data);
     } else {
         // stream-ordered release: later work on the compute stream may reuse the block immediately
-        give_block(gpu_context(device.index), data, block);
+        give_block(gpu_context(device.index), data, block, captured);
     }
 }
 
@@ -164,7 +166,7 @@ std::shared_ptr<Storage> allocate_storage(std::size_t bytes, Device device) {
         std::memset(storage->data, 0, rounded);
     } else {
         storage->block = rounded;
-        storage->data = take_block(gpu_context(device.index), storage->block);
+        storage->data = take_block(gpu_context(device.index), storage->block, storage->captured);
     }
     return storage;
 }

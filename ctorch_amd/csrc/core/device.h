@@ -23,8 +23,8 @@ void hip_check(int status, const char* what);
 /// the runtime's pool and back: a hipMallocAsync / hipFreeAsync pair takes the host 10.6 us on MI355X, and a small decoder
 /// chunk allocates ten tensors.  A block freed while work that uses it is still queued may be handed out at
 /// once, as the runtime's pool does, because all of a device's work is ordered on its one compute stream.  While that
-/// stream is being captured nothing is taken from here or put back.  At most `limit` bytes and kBlocks blocks are held;
-/// the oldest go back to the runtime's pool.
+/// stream is being captured nothing is taken from here or put back, and a block that was allocated then never comes
+/// here: it is the graph's.  At most `limit` bytes and kBlocks blocks are held; the oldest go back to the runtime's pool.
 struct BlockCache {
     static constexpr std::size_t kBlockMax = std::size_t(32) << 20, kLimit = std::size_t(256) << 20, kBlocks = 256;
     struct Block {
@@ -55,6 +55,7 @@ struct Storage {
     void* data = nullptr;
     std::size_t bytes = 0;
     std::size_t block = 0; ///< GPU: bytes of the block behind it
+    bool captured = false; ///< GPU: allocated while the stream was captured
     Device device{};
     Storage() = default;
     Storage(const Storage&) = delete;

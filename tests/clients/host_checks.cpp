@@ -3,6 +3,8 @@
 // tests/test_host_rules.py.
 //
 //   host_checks split BATCH HEADS KV_HEADS HEAD_DIM KV_BF16 LENGTH SOURCE CAUSAL    attention_split: splits, keys per split
+//   host_checks capture                         a block allocated while the stream is captured and freed after it: how many
+//                                               went back to the runtime, and 1 if the next allocation got it again
 //   host_checks workspace ENTRY ROWS K BYTES    launches of linear, swiglu or attention over bf16 weights with BYTES of
 //                                               device memory left for their workspaces (-1: no limit)
 #include "dl/decoder.h"
@@ -25,7 +27,7 @@ namespace {
 struct Device {
     std::map<void*, size_t> blocks; // allocations alive
     size_t used = 0, peak = 0, limit = SIZE_MAX, launches = 0;
-    int last_error = 0;
+    int last_error = 0, capturing = 0;
 } fake;
 
 } // namespace
@@ -70,7 +72,7 @@ int dlh_event_record(dlh_event, dlh_stream) { return 0; }
 int dlh_event_synchronize(dlh_event) { return 0; }
 int dlh_event_elapsed(dlh_event, dlh_event, float* ms) { return *ms = 0, 0; }
 int dlh_capture_begin(dlh_stream) { return 0; }
-int dlh_stream_capturing(dlh_stream, int* capturing) { return *capturing = 0, 0; }
+int dlh_stream_capturing(dlh_stream, int* capturing) { return *capturing = fake.capturing, 0; }
 int dlh_capture_end(dlh_stream, dlh_graph*) { return 0; }
 int dlh_graph_launch(dlh_graph, dlh_stream) { return 0; }
 int dlh_graph_destroy(dlh_graph) { return 0; }
@@ -109,6 +111,22 @@ int split(char** arg) {
     return 0;
 }
 
+int capture() {
+    const dl::Device gpu = dl::Device::gpu(0);
+    const dl::Index n = 1 << 20;
+    { dl::Tensor first = empty_tensor({64}, dl::DType::f32, gpu); } // the context exists
+    fake.capturing = 1;
+    dl::Tensor recorded = empty_tensor({n}, dl::DType::f32, gpu);
+    fake.capturing = 0;
+    void* block = dl::detail::mutable_data(recorded);
+    const size_t alive = fake.blocks.size();
+    recorded = dl::Tensor();
+    const size_t returned = alive - fake.blocks.size();
+    const dl::Tensor next = empty_tensor({n}, dl::DType::f32, gpu);
+    std::printf("%zu %d\n", returned, !returned && dl::detail::mutable_data(next) == block);
+    return 0;
+}
+
 int workspace(char** arg) {
     const std::string entry = arg[0];
     const dl::Index rows = std::atoll(arg[1]), k = std::atoll(arg[2]), left = std::atoll(arg[3]);
@@ -142,6 +160,7 @@ int workspace(char** arg) {
 int main(int argc, char** argv) {
     try {
         if (argc == 10 && std::strcmp(argv[1], "split") == 0) return split(argv + 2);
+        if (argc == 2 && std::strcmp(argv[1], "capture") == 0) return capture();
         if (argc == 6 && std::strcmp(argv[1], "workspace") == 0) return workspace(argv + 2);
     } catch (const std::exception& error) {
         std::fprintf(stderr, "%s\n", error.what());

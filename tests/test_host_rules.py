@@ -45,3 +45,9 @@ def test_no_staged_copy_past_4_gib_of_rows(entry):
     # the buffers are reserved, not touched
     few, many = (int(checks("workspace", entry, rows, 4096, -1)) for rows in (1 << 18, (1 << 18) + 1))
     assert few < 20 and many >= (1 << 18) // 64
+
+
+def test_a_block_of_a_captured_graph_is_not_handed_out_again():
+    # it belongs to the graph's allocation node: a free returns it to the runtime, also after the capture has ended
+    returned, reused = map(int, checks("capture").split())
+    assert returned == 1 and not reused
