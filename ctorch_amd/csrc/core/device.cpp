@@ -135,12 +135,9 @@ void give_block(GpuContext& context, void* data, std::size_t bytes, bool capture
         } catch (const std::bad_alloc&) {
         }
     }
-    if (!kept) {
-        (void)dlh_free_async(data, context.stream);
-        return;
-    }
-    cache.held += bytes;
-    shrink(context, cache.limit, BlockCache::kBlocks);
+    if (kept) cache.held += bytes;
+    else (void)dlh_free_async(data, context.stream);
+    if (!direct) shrink(context, cache.limit, BlockCache::kBlocks);
 }
 
 } // namespace
@@ -213,7 +210,8 @@ void set_memory_release_threshold(std::uint64_t bytes, int device) {
     {
         std::lock_guard<std::mutex> lock(context.cache.mutex);
         context.cache.limit = static_cast<std::size_t>(std::min<std::uint64_t>(bytes, detail::BlockCache::kLimit));
-        detail::shrink(context, context.cache.limit, detail::BlockCache::kBlocks);
+        // during a capture the next free after it brings the held blocks within the limit
+        if (!detail::capturing(context)) detail::shrink(context, context.cache.limit, detail::BlockCache::kBlocks);
     }
     detail::hip_check(dlh_pool_set_threshold(device, bytes), "pool release threshold");
 }
@@ -229,6 +227,7 @@ void reset_peak_memory_stats(int device) {
 
 void release_unused_memory(int device) {
     auto& context = detail::gpu_context(device);
+    detail::hip_check(dlh_stream_synchronize(context.stream), "synchronize"); // refused during a capture
     {
         std::lock_guard<std::mutex> lock(context.cache.mutex);
         detail::shrink(context, 0, 0);

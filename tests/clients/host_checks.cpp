@@ -5,6 +5,8 @@
 //   host_checks split BATCH HEADS KV_HEADS HEAD_DIM KV_BF16 LENGTH SOURCE CAUSAL    attention_split: splits, keys per split
 //   host_checks capture                         a block allocated while the stream is captured and freed after it: how many
 //                                               went back to the runtime, and 1 if the next allocation got it again
+//   host_checks capture_release                blocks that went back to the runtime: during a capture by a threshold of 0 and
+//                                               by release_unused_memory, and by the next free after the capture
 //   host_checks workspace ENTRY ROWS K BYTES    launches of linear, swiglu or attention over bf16 weights with BYTES of
 //                                               device memory left for their workspaces (-1: no limit)
 #include "dl/decoder.h"
@@ -42,7 +44,7 @@ int dlh_get_device(int* device) { return *device = 0, 0; }
 int dlh_device_properties_get(int, dlh_device_properties* out) { return std::memset(out, 0, sizeof(*out)), 0; }
 int dlh_stream_create(dlh_stream* stream) { return *stream = reinterpret_cast<dlh_stream>(&fake), 0; }
 int dlh_stream_destroy(dlh_stream) { return 0; }
-int dlh_stream_synchronize(dlh_stream) { return 0; }
+int dlh_stream_synchronize(dlh_stream) { return fake.capturing ? hipErrorStreamCaptureUnsupported : 0; }
 int dlh_pool_configure(int) { return 0; }
 int dlh_malloc_async(void** pointer, size_t bytes, dlh_stream) {
     if (bytes > fake.limit - std::min(fake.limit, fake.used)) return fake.last_error = hipErrorOutOfMemory;
@@ -127,6 +129,23 @@ int capture() {
     return 0;
 }
 
+int capture_release() {
+    { dl::Tensor held = empty_tensor({1 << 20}, dl::DType::f32, dl::Device::gpu(0)); }
+    const size_t all = fake.blocks.size();
+    fake.capturing = 1;
+    dl::gpu::set_memory_release_threshold(0);
+    const size_t by_threshold = all - fake.blocks.size();
+    try {
+        dl::gpu::release_unused_memory(); // refused: it waits for the stream
+    } catch (const std::runtime_error&) {
+    }
+    const size_t by_release = all - fake.blocks.size();
+    fake.capturing = 0;
+    { dl::Tensor next = empty_tensor({64}, dl::DType::f32, dl::Device::gpu(0)); }
+    std::printf("%zu %zu %zu\n", by_threshold, by_release, all - fake.blocks.size());
+    return 0;
+}
+
 int workspace(char** arg) {
     const std::string entry = arg[0];
     const dl::Index rows = std::atoll(arg[1]), k = std::atoll(arg[2]), left = std::atoll(arg[3]);
@@ -161,6 +180,7 @@ int main(int argc, char** argv) {
     try {
         if (argc == 10 && std::strcmp(argv[1], "split") == 0) return split(argv + 2);
         if (argc == 2 && std::strcmp(argv[1], "capture") == 0) return capture();
+        if (argc == 2 && std::strcmp(argv[1], "capture_release") == 0) return capture_release();
         if (argc == 6 && std::strcmp(argv[1], "workspace") == 0) return workspace(argv + 2);
     } catch (const std::exception& error) {
         std::fprintf(stderr, "%s\n", error.what());

@@ -51,3 +51,8 @@ def test_a_block_of_a_captured_graph_is_not_handed_out_again():
     # it belongs to the graph's allocation node: a free returns it to the runtime, also after the capture has ended
     returned, reused = map(int, checks("capture").split())
     assert returned == 1 and not reused
+
+
+def test_held_blocks_are_not_freed_into_a_capture():
+    # a free during a capture becomes a node of the graph, and each replay would free the block again
+    assert checks("capture_release").split() == ["0", "0", "1"]
