@@ -135,7 +135,7 @@ void give_block(GpuContext& context, void* data, std::size_t bytes, bool capture
         } catch (const std::bad_alloc&) {
         }
     }
-    if (kept) cache.held += bytes;
+    if (kept) cache.held_peak = std::max(cache.held_peak, cache.held += bytes);
     else (void)dlh_free_async(data, context.stream);
     if (!direct) shrink(context, cache.limit, BlockCache::kBlocks);
 }
@@ -201,7 +201,11 @@ MemoryStats memory_stats(int device) {
     // held blocks are free ones: `used` counts the live tensors and what others have of the pool
     const std::uint64_t ours = cache.live + cache.held, others = out.used_bytes > ours ? out.used_bytes - ours : 0;
     out.used_bytes = cache.live + others;
-    out.peak_used_bytes = cache.peak > 0 ? cache.peak + others : 0;
+    // Their peak: that of the tensors with what others have now, or the pool's own less the most that was held, the larger
+    // (others may have given back what they had at the pool's peak)
+    const std::uint64_t pool_peak = out.peak_used_bytes;
+    out.peak_used_bytes = std::max<std::uint64_t>(cache.peak > 0 ? cache.peak + others : 0,
+                                                  pool_peak > cache.held_peak ? pool_peak - cache.held_peak : 0);
     return out;
 }
 
@@ -221,6 +225,7 @@ void reset_peak_memory_stats(int device) {
     {
         std::lock_guard<std::mutex> lock(cache.mutex);
         cache.peak = 0; // the next allocation raises it again
+        cache.held_peak = cache.held;
     }
     detail::hip_check(dlh_pool_reset_peaks(device), "pool peak reset");
 }

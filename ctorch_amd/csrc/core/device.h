@@ -35,6 +35,7 @@ struct BlockCache {
     std::multimap<std::size_t, Block> blocks; ///< by size
     std::size_t held = 0, limit = kLimit;
     std::size_t live = 0, peak = 0; ///< bytes of the tensors alive now, and their high-water mark
+    std::size_t held_peak = 0;      ///< most bytes held at once since the peaks were reset
     std::uint64_t clock = 0;
 };
 

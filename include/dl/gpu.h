@@ -11,7 +11,8 @@ namespace dl::gpu {
 
 /// Bytes of the device's pool.  `used` counts live allocations, `reserved` (as the HIP runtime reports it) adds the
 /// free blocks kept for reuse, among them up to 256 MiB of small ones that the library hands out again itself; pinned
-/// host memory and the HIP runtime's own allocations are not counted.
+/// host memory and the HIP runtime's own allocations are not counted.  The peak of `used` may fall short by what was held
+/// of those, where other users of the pool set it.
 struct MemoryStats {
     std::uint64_t used_bytes, reserved_bytes;
     std::uint64_t peak_used_bytes, peak_reserved_bytes;

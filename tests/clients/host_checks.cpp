@@ -7,6 +7,9 @@
 //                                               went back to the runtime, and 1 if the next allocation got it again
 //   host_checks capture_release                blocks that went back to the runtime: during a capture by a threshold of 0 and
 //                                               by release_unused_memory, and by the next free after the capture
+//   host_checks peak                            MiB of memory_stats' used and peak with a tensor of 4 alive: after another
+//                                               user of the pool had 64 and gave them back, with the tensor then freed and
+//                                               held, and after a reset
 //   host_checks workspace ENTRY ROWS K BYTES    launches of linear, swiglu or attention over bf16 weights with BYTES of
 //                                               device memory left for their workspaces (-1: no limit)
 #include "dl/decoder.h"
@@ -66,7 +69,7 @@ int dlh_pool_stats(int, uint64_t* used, uint64_t* reserved, uint64_t* peak_used,
 }
 int dlh_pool_trim(int) { return 0; }
 int dlh_pool_set_threshold(int, uint64_t) { return 0; }
-int dlh_pool_reset_peaks(int) { return fake.peak = fake.used, 0; }
+int dlh_pool_reset_peaks(int) { return fake.peak = 0, 0; } // the next allocation raises it again
 int dlh_memcpy_async(void* to, const void* from, size_t bytes, int, dlh_stream) { return std::memcpy(to, from, bytes), 0; }
 int dlh_event_create(dlh_event*) { return 0; }
 int dlh_event_destroy(dlh_event) { return 0; }
@@ -146,6 +149,25 @@ int capture_release() {
     return 0;
 }
 
+int peak() {
+    const dl::Device gpu = dl::Device::gpu(0);
+    dl::Tensor own = empty_tensor({1 << 20}, dl::DType::f32, gpu);
+    auto print = [] {
+        const auto stats = dl::gpu::memory_stats(0);
+        std::printf("%llu %llu\n", static_cast<unsigned long long>(stats.used_bytes >> 20),
+                    static_cast<unsigned long long>(stats.peak_used_bytes >> 20));
+    };
+    void* others = nullptr;
+    (void)dlh_malloc_async(&others, size_t(64) << 20, nullptr);
+    (void)dlh_free_async(others, nullptr);
+    print();
+    own = dl::Tensor();
+    print();
+    dl::gpu::reset_peak_memory_stats(0);
+    print();
+    return 0;
+}
+
 int workspace(char** arg) {
     const std::string entry = arg[0];
     const dl::Index rows = std::atoll(arg[1]), k = std::atoll(arg[2]), left = std::atoll(arg[3]);
@@ -181,6 +203,7 @@ int main(int argc, char** argv) {
         if (argc == 10 && std::strcmp(argv[1], "split") == 0) return split(argv + 2);
         if (argc == 2 && std::strcmp(argv[1], "capture") == 0) return capture();
         if (argc == 2 && std::strcmp(argv[1], "capture_release") == 0) return capture_release();
+        if (argc == 2 && std::strcmp(argv[1], "peak") == 0) return peak();
         if (argc == 6 && std::strcmp(argv[1], "workspace") == 0) return workspace(argv + 2);
     } catch (const std::exception& error) {
         std::fprintf(stderr, "%s\n", error.what());

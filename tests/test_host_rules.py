@@ -56,3 +56,10 @@ def test_a_block_of_a_captured_graph_is_not_handed_out_again():
 def test_held_blocks_are_not_freed_into_a_capture():
     # a free during a capture becomes a node of the graph, and each replay would free the block again
     assert checks("capture_release").split() == ["0", "0", "1"]
+
+
+def test_the_peak_keeps_what_others_had_of_the_pool():
+    alive, held, reset = (tuple(map(int, line.split())) for line in checks("peak").splitlines())
+    assert alive == (4, 68)
+    assert held[0] == 0 and 64 <= held[1] <= 68  # at most the held blocks too little
+    assert reset == (0, 0)
