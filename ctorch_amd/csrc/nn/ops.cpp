@@ -122,6 +122,11 @@ void attention_split(Index batch, Index heads, Index kv_heads, Index head_dim, b
     if (causal && dlk_attention_prefill_heads(static_cast<int>(heads), static_cast<int>(kv_heads),
                                               static_cast<int>(head_dim), static_cast<int>(length)))
         return;
+    // Head sizes below 16 (attention_small: a wave per query row, and a merge that takes a work-group per row): splits
+    // pay where a row's keys are long against the number of rows.  Measured on MI355X, 4 sequences of 32 / 8 heads, us
+    // whole / split: head size 2, 8192 rows over 256 keys 14 / 152, 2048 over 4096 51 / 70, 1024 over 4096 47 / 40; head
+    // size 8, 4096 over 1024 66 / 79, 1024 over 4096 121 / 71, 512 over 1024 30 / 18.
+    if (head_dim < 16 && source * head_dim < 8 * batch * heads * length) return;
     // the others (attention_rows, a work-group per 64 rows of a KV head): key splits of two or more 64-key tiles until
     // every CU has a work-group.  Measured on MI355X at 4 sequences x 7 positions over 1508 keys (32 such groups), us a
     // layer with its merge: 8 splits 16.3, 12 17.2, 24 (one tile each) 17.4; with 256 groups already (4 x 510 byte

@@ -131,3 +131,19 @@ def test_empty_queries_and_chunks_are_refused_and_leave_the_cache(batch, length,
         with pytest.raises(ct.DLError):
             ct.decode(decoder, empty, cache)
         assert cache.length == 3
+
+
+@pytest.mark.parametrize("D", [2, 4, 8])
+@pytest.mark.parametrize("B,H,KV,L,S", [(2, 8, 2, 64, 65), (1, 4, 4, 5, 700), (2, 6, 3, 17, 130)])
+def test_small_heads_with_and_without_key_splits(D, B, H, KV, L, S):
+    say(f"case: attention B={B} H={H} KV={KV} L={L} S={S} D={D}")
+    rng = np.random.default_rng(S + D)
+    q = rng.standard_normal((B, H, L, D)).astype(np.float32)
+    k, v = (rng.standard_normal((B, KV, S, D)).astype(np.float32) for _ in range(2))
+    mask = rng.random((B, 1, L, S)) < 0.5
+    mask[..., 0] = True
+    for m in (None, mask):
+        got = ct.grouped_query_attention(*(ct.Tensor.from_numpy(a, ct.F32, GPU) for a in (q, k, v)),
+                                         None if m is None else ct.Tensor.from_numpy(m, ct.BOOL, GPU)).numpy()
+        want = reference(q, k, v, m)
+        assert np.linalg.norm(got - want) <= 2.0**-24 * (np.sqrt(D) + np.sqrt(S) + 8) * np.linalg.norm(want)

@@ -63,3 +63,12 @@ def test_the_peak_keeps_what_others_had_of_the_pool():
     assert alive == (4, 68)
     assert held[0] == 0 and 64 <= held[1] <= 68  # at most the held blocks too little
     assert reset == (0, 0)
+
+
+@pytest.mark.parametrize("head_dim,length,source,split_up", [
+    (2, 64, 256, False), (2, 32, 4096, False), (2, 16, 1024, False), (4, 64, 4096, False), (8, 64, 1024, False),
+    (8, 32, 1024, False), (2, 4, 4096, True), (2, 8, 16384, True), (8, 8, 4096, True), (8, 4, 1024, True)])
+def test_many_rows_of_small_heads_are_not_split(head_dim, length, source, split_up):
+    # 4 sequences, 32 / 8 heads: a wave per query row, so many rows fill the device without key splits and their merge
+    splits, chunk = split(4, 32, 8, head_dim, False, length, source, False)
+    assert (splits > 1) == split_up and splits * chunk >= source
