@@ -502,15 +502,19 @@ int launch_combine(const dlk_attention_params& p, hipStream_t stream) {
     return static_cast<int>(hipGetLastError());
 }
 
-// The fewest row tiles per work-group that hold the rows of a KV head: the waves left over share the keys.
-template <typename KT, int HD>
-int launch(const dlk_attention_params& p, hipStream_t stream) {
-    const int group = p.H / p.KV, rows = group * p.L;
-    int wr = rows <= 16 ? 1 : rows <= 32 ? 2 : 4;
+// Row tiles per work-group: the fewest that hold the rows of a KV head, and the waves left over share the keys.
+int row_tiles(const dlk_attention_params& p) {
+    const int rows = p.H / p.KV * p.L;
+    if (rows <= 32) return rows <= 16 ? 1 : 2;
     // four row tiles that leave a CU with less than two work-groups: two, so that one's products run under another's
     // staging and softmax (4 x 510 causal positions, 8 / 2 heads of 32: 18.5 us at 256 work-groups, 15.2 at 512, 16.8 at
     // 1024 of one row tile; 4 x 500 positions of 32 / 8 heads of 64: 111 at 1024, 120 at 2048)
-    if (wr == 4 && static_cast<int64_t>((rows + 63) / 64) * p.splits * p.B * p.KV < 512) wr = 2;
+    return static_cast<int64_t>((rows + 63) / 64) * p.splits * p.B * p.KV < 512 ? 2 : 4;
+}
+
+template <typename KT, int HD>
+int launch(const dlk_attention_params& p, hipStream_t stream) {
+    const int group = p.H / p.KV, rows = group * p.L, wr = row_tiles(p);
     const dim3 grid(p.splits, (rows + 16 * wr - 1) / (16 * wr), p.B * p.KV);
     const dim3 threads(kThreads);
     if (wr == 1) hipLaunchKernelGGL((attention_rows<KT, HD, 1>), grid, threads, 0, stream, p, group);
@@ -553,6 +557,14 @@ extern "C" int dlk_attention_scratch(int device, float** address) {
     }
     *address = addresses[device];
     return 0;
+}
+
+extern "C" const char* dlk_attention_kernel(const dlk_attention_params* p) {
+    if (dlk_attention_matrix_eligible(p)) return "matrix";
+    if (dlk_attention_prefill_eligible(p)) return "prefill";
+    if (p->hd < 16) return "small";
+    const int tiles = dlk::row_tiles(*p);
+    return tiles == 1 ? "rows 1" : tiles == 2 ? "rows 2" : "rows 4";
 }
 
 extern "C" int dlk_attention_takes_strides(const dlk_attention_params* p) {

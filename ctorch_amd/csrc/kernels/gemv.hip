@@ -98,6 +98,14 @@ int launch_reduce(dlk_gemv_params& p, int splits, hipStream_t stream) {
                                             dim3(kReduceThreads), args, 0, stream));
 }
 
+enum class Route { gemv, rows, narrow, mid, tiles, f32 };
+
+/// The kernel that dlk_gemv launches.
+Route route_of(const dlk_gemv_params& p) {
+    if (staged(p)) return dlk_tiles_kernel_narrow(p).fn ? Route::narrow : use_mid(p) ? Route::mid : Route::tiles;
+    return dlk::gemm::eligible(p) ? Route::rows : dlk::gemm32::eligible(p) ? Route::f32 : Route::gemv;
+}
+
 int launch_prepare(const dlk_gemv_params& p, hipStream_t stream);
 
 // The staged rows through gemm_mid, and the sum of its key slices.
@@ -126,16 +134,15 @@ int launch_mid(const dlk_gemv_params& params, hipStream_t stream) {
 
 // Tiled path: prepare_rows splits the activation rows into the staging workspace (unless the caller says it
 // already holds them), then the tiled projection.
-int launch_tiles(const dlk_gemv_params& p, hipStream_t stream) {
+int launch_tiles(const dlk_gemv_params& p, Route route, hipStream_t stream) {
     using namespace dlk::tiles;
-    const Kernel narrow = dlk_tiles_kernel_narrow(p);
-    const Kernel kernel = narrow.fn ? narrow : resolve_tiles(p);
+    const Kernel kernel = route == Route::narrow ? dlk_tiles_kernel_narrow(p) : resolve_tiles(p);
     if (!kernel.fn) return static_cast<int>(hipErrorInvalidValue);
     const int status = launch_prepare(p, stream);
     if (status != 0) return status;
     void* args[] = {const_cast<dlk_gemv_params*>(&p)};
-    if (!narrow.fn && use_mid(p)) return launch_mid(p, stream);
-    if (narrow.fn) {
+    if (route == Route::mid) return launch_mid(p, stream);
+    if (route == Route::narrow) {
         const int waves = (p.M + 15) / 16;
         return static_cast<int>(hipLaunchKernel(kernel.fn, dim3((waves + kNarrowWaves - 1) / kNarrowWaves),
                                                 dim3(kNarrowWaves * dlk::kWave), args, 0, stream));
@@ -332,13 +339,26 @@ extern "C" int dlk_gemv_uses_rows(const dlk_gemv_params* p) {
     return !staged(*p) && dlk::gemm::eligible(*p) ? 1 : 0;
 }
 
+extern "C" const char* dlk_gemv_kernel(const dlk_gemv_params* p) {
+    static constexpr const char* shapes[] = {"f32 128x128", "f32 64x64", "f32 64x32", "f32 32x16"};
+    switch (route_of(*p)) {
+    case Route::rows: return "rows";
+    case Route::narrow: return "narrow";
+    case Route::mid: return "mid";
+    case Route::tiles: return "tiles";
+    case Route::f32: return shapes[dlk::gemm32::shape_of(*p)];
+    default: return "gemv";
+    }
+}
+
 extern "C" int dlk_gemv_folds_lora(const dlk_gemv_params* p) {
     return !staged(*p) && dlk::gemm::eligible(*p) && dlk::gemm::lora_fold_eligible(*p) ? 1 : 0;
 }
 
 extern "C" int64_t dlk_gemv_split_floats(const dlk_gemv_params* p) {
-    if (staged(*p)) return !dlk_tiles_kernel_narrow(*p).fn && use_mid(*p) ? dlk::mid::split_floats(*p) : 0;
-    if (!dlk::gemm::eligible(*p)) return 0;
+    const Route route = route_of(*p);
+    if (route == Route::mid) return dlk::mid::split_floats(*p);
+    if (route != Route::rows) return 0;
     const int rows = std::min(p->M, dlk::gemm::kMaxRows);
     return dlk::gemm::split_floats(*p, dlk::gemm::splits_of(*p, rows), rows);
 }
@@ -388,9 +408,10 @@ extern "C" int dlk_gemv(const dlk_gemv_params* params, dlh_stream stream_handle)
     // only the wide kernel applies LoRA down rows
     if ((params->lora_down[0] || params->lora_down[1] || params->lora_down[2]) && !dlk_gemv_folds_lora(params))
         return static_cast<int>(hipErrorInvalidValue);
-    if (staged(*params)) return launch_tiles(*params, stream);
-    if (dlk::gemm::eligible(*params)) return launch_gemm(*params, stream);
-    if (dlk::gemm32::eligible(*params)) return launch_f32(*params, stream);
+    const Route route = route_of(*params);
+    if (route == Route::rows) return launch_gemm(*params, stream);
+    if (route == Route::f32) return launch_f32(*params, stream);
+    if (route != Route::gemv) return launch_tiles(*params, route, stream);
     const int waves = launch_waves(*params);
     if (waves <= 0) return static_cast<int>(hipErrorInvalidValue);
     const int blocks = (waves + kWavesPerBlock - 1) / kWavesPerBlock;

@@ -109,6 +109,9 @@ typedef struct dlk_gemv_params {
    tile t interleaves gate and up rows 8 t .. +8 (tile row 2 j: gate 8 t + j, 2 j + 1: up 8 t + j).  out holds
    rows * K (swiglu: 2 * rows * K) bf16. */
 int dlk_pack_tiles(const void* w0, const void* w1, int swiglu, int64_t rows, int64_t K, void* out, dlh_stream stream);
+/* The kernel that dlk_gemv launches for these parameters: "gemv", "rows" (gemm_rows or gemm_wide), "narrow", "mid" or
+   "tiles" (the staged ones), or "f32 " and its work-group shape. */
+const char* dlk_gemv_kernel(const dlk_gemv_params* p);
 /* 1 when dlk_gemv takes a batched matrix-core kernel (gemm_rows or gemm_wide, which read w_tiles) for this
    launch. */
 int dlk_gemv_uses_rows(const dlk_gemv_params* p);
@@ -202,6 +205,9 @@ int dlk_attention_matrix_heads(int heads, int kv_heads, int head_dim);
 
 
 int dlk_attention(const dlk_attention_params* p, dlh_stream stream);
+/* The kernel that dlk_attention launches for these parameters: "matrix", "prefill", "small", or "rows" and its row tiles
+   per work-group. */
+const char* dlk_attention_kernel(const dlk_attention_params* p);
 /* 1 when dlk_attention takes the general kernel for these parameters, which reads the query through its strides. */
 int dlk_attention_takes_strides(const dlk_attention_params* p);
 /* Floats of the device-resident scratch array behind the allocation-free attention entry (8 MiB per GPU). */

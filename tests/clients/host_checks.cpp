@@ -3,6 +3,12 @@
 // tests/test_host_rules.py.
 //
 //   host_checks split BATCH HEADS KV_HEADS HEAD_DIM KV_BF16 LENGTH SOURCE CAUSAL    attention_split: splits, keys per split
+//   host_checks projection EPILOGUE ROWS K R0 R1 R2 BF16 BIAS LAYER
+//                                               the kernel of a projection (store, residual, qkv or swiglu) with R0, R1, R2
+//                                               weight rows (0: no segment): in a decoder layer, or called by itself
+//   host_checks attention BATCH HEADS KV_HEADS HEAD_DIM KV_BF16 LENGTH SOURCE CAUSAL MASKED    the kernel of an attention
+//   host_checks threshold                       blocks held after a free: at first, at threshold 0, back at the first one
+//   host_checks retry                           allocations that the memory holds only without the held blocks: 1, 1
 //   host_checks capture                         a block allocated while the stream is captured and freed after it: how many
 //                                               went back to the runtime, and 1 if the next allocation got it again
 //   host_checks capture_release                blocks that went back to the runtime: during a capture by a threshold of 0 and
@@ -116,6 +122,90 @@ int split(char** arg) {
     return 0;
 }
 
+int projection(char** arg) {
+    const std::string epilogue = arg[0];
+    auto at = [&](int i) { return static_cast<int>(std::atoll(arg[i])); };
+    alignas(64) static char memory[64]; // every address that the rules look at; nothing is launched
+    auto* f32 = reinterpret_cast<float*>(memory);
+    dlk_gemv_params p{};
+    p.epilogue = epilogue == "store" ? DLK_EPI_STORE : epilogue == "residual" ? DLK_EPI_RESIDUAL
+               : epilogue == "qkv" ? DLK_EPI_QKV : DLK_EPI_SWIGLU;
+    p.M = at(1), p.K = at(2), p.ldx = p.K, p.x = f32, p.y = f32;
+    for (int s = 0; s < 3 && at(3 + s) > 0; ++s) {
+        p.seg_rows[p.nseg++] = at(3 + s);
+        p.w[s] = memory;
+        if (p.epilogue != DLK_EPI_SWIGLU || s == 0) p.ldy += p.epilogue == DLK_EPI_QKV && s > 0 ? 0 : at(3 + s);
+    }
+    p.w_bf16 = at(6);
+    p.bias = at(7) ? memory : nullptr;
+    p.residual = f32, p.ldres = p.ldy;
+    p.head_dim = 32, p.kv_heads = 1, p.length = p.M, p.acc_scale = 1.0f;
+    p.k_cache = p.v_cache = memory;
+    p.cosine = p.sine = f32;
+    p.apply_norm = p.epilogue == DLK_EPI_QKV || p.epilogue == DLK_EPI_SWIGLU;
+    if (at(8) || dlk_gemv_uses_rows(&p)) { // what attach_workspace and attach_workspace_if_room attach
+        p.stage_bytes = dlk_gemv_stage_bytes(&p);
+        p.stage = p.stage_bytes > 0 ? memory : nullptr;
+    }
+    std::printf("%s\n", dlk_gemv_kernel(&p));
+    return 0;
+}
+
+int attention(char** arg) {
+    auto at = [&](int i) { return static_cast<int>(std::atoll(arg[i])); };
+    alignas(64) static char memory[64];
+    dlk_attention_params p{};
+    p.B = at(0), p.H = at(1), p.KV = at(2), p.hd = at(3), p.kv_bf16 = at(4), p.L = at(5), p.causal = at(7);
+    p.capacity = at(6), p.first_host = at(6) - at(5), p.early_keys = at(6);
+    p.q = p.out = reinterpret_cast<float*>(memory);
+    p.k = p.v = memory;
+    p.ldq = p.ldo = static_cast<int64_t>(p.H) * p.hd;
+    p.keep_mask = at(8) ? reinterpret_cast<unsigned char*>(memory) : nullptr;
+    dl::detail::attention_split(p.B, p.H, p.KV, p.hd, p.kv_bf16 != 0, p.L, p.capacity, p.causal != 0, p.splits, p.chunk);
+    std::printf("%s\n", dlk_attention_kernel(&p));
+    return 0;
+}
+
+int threshold() {
+    const dl::Device gpu = dl::Device::gpu(0);
+    { dl::Tensor first = empty_tensor({64}, dl::DType::f32, gpu); }
+    dl::gpu::release_unused_memory(0);
+    const size_t base = fake.blocks.size();
+    auto held = [&] {
+        { dl::Tensor t = empty_tensor({1 << 18}, dl::DType::f32, gpu); }
+        return fake.blocks.size() - base;
+    };
+    const size_t before = held();
+    dl::gpu::set_memory_release_threshold(0);
+    const size_t at_once = fake.blocks.size() - base, at_zero = held();
+    dl::gpu::set_memory_release_threshold(UINT64_MAX);
+    std::printf("%zu %zu %zu %zu\n", before, at_once, at_zero, held());
+    return 0;
+}
+
+int retry() {
+    const dl::Device gpu = dl::Device::gpu(0);
+    const dl::Index mib = 1 << 18; // floats
+    auto hold = [&] { // 3 x 16 MiB, freed
+        dl::Tensor a = empty_tensor({16 * mib}, dl::DType::f32, gpu), b = empty_tensor({16 * mib}, dl::DType::f32, gpu),
+                   c = empty_tensor({16 * mib}, dl::DType::f32, gpu);
+    };
+    hold();
+    fake.limit = fake.used + (size_t(8) << 20);
+    int fits[2];
+    for (int i = 0; i < 2; ++i) { // above the largest block that is held, and below it
+        try {
+            dl::Tensor t = empty_tensor({(i == 0 ? 40 : 24) * mib}, dl::DType::f32, gpu);
+            fits[i] = 1;
+        } catch (const std::runtime_error&) {
+            fits[i] = 0;
+        }
+        hold();
+    }
+    std::printf("%d %d\n", fits[0], fits[1]);
+    return 0;
+}
+
 int capture() {
     const dl::Device gpu = dl::Device::gpu(0);
     const dl::Index n = 1 << 20;
@@ -201,6 +291,10 @@ int workspace(char** arg) {
 int main(int argc, char** argv) {
     try {
         if (argc == 10 && std::strcmp(argv[1], "split") == 0) return split(argv + 2);
+        if (argc == 11 && std::strcmp(argv[1], "projection") == 0) return projection(argv + 2);
+        if (argc == 11 && std::strcmp(argv[1], "attention") == 0) return attention(argv + 2);
+        if (argc == 2 && std::strcmp(argv[1], "threshold") == 0) return threshold();
+        if (argc == 2 && std::strcmp(argv[1], "retry") == 0) return retry();
         if (argc == 2 && std::strcmp(argv[1], "capture") == 0) return capture();
         if (argc == 2 && std::strcmp(argv[1], "capture_release") == 0) return capture_release();
         if (argc == 2 && std::strcmp(argv[1], "peak") == 0) return peak();

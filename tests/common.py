@@ -114,3 +114,13 @@ def greedy_steps(ref, gpu, rc, gc, ids, steps, label):
         assert gap <= 2e-2, (label, step)
         ids = want.argmax(-1).reshape(-1, 1)
     return ids
+
+
+def agree(got: np.ndarray, want: np.ndarray, bound: float) -> None:
+    """The 2-norm of the error against that of the 64-bit result: of the whole, and at twice the bound of every row and
+    column of a matrix (an error in an edge tile is not averaged away over the rest)."""
+    error = got.astype(np.float64) - want
+    assert np.linalg.norm(error) <= bound * np.linalg.norm(want)
+    for axis in range(want.ndim):
+        off, size = np.linalg.norm(error, axis=axis), np.linalg.norm(want, axis=axis)
+        assert np.all(off <= 2 * bound * size), (axis, int(np.argmax(off / size)), float(np.max(off / size)))

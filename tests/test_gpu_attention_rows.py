@@ -57,6 +57,35 @@ def test_attention_rows_match_64_bit_results(B, H, KV, L, S, D, bf16, masked):
         assert np.linalg.norm(error) <= 2.0**-24 * (np.sqrt(D) + np.sqrt(S) + 8) * np.linalg.norm(np.nan_to_num(want))
 
 
+# B, H, KV, L, S, D, kernel: 64 query rows to a work-group, a wave to each 16
+MANY = [(4, 32, 8, 270, 275, D, "rows 4") for D in (16, 32, 64, 128)]
+
+
+@pytest.mark.parametrize("bf16,masked", [(False, False), (False, True), (True, True)])
+@pytest.mark.parametrize("B,H,KV,L,S,D,kernel", MANY)
+def test_attention_over_many_rows_matches_64_bit_results(B, H, KV, L, S, D, kernel, bf16, masked):
+    say(f"case: attention B={B} H={H} KV={KV} L={L} S={S} D={D} bf16={bf16} masked={masked} ({kernel})")
+    rng = np.random.default_rng(D)
+    q = rng.standard_normal((B, H, L, D)).astype(np.float32)
+    k, v = (rng.standard_normal((B, KV, S, D)).astype(np.float32) for _ in range(2))
+    encode = oracle.bf16_encode if bf16 else (lambda a: a)
+    gk, gv = (ct.Tensor.from_numpy(encode(a), ct.BF16 if bf16 else ct.F32, GPU) for a in (k, v))
+    if bf16:
+        k, v = (oracle.bf16_decode(encode(a)) for a in (k, v))
+    mask = None
+    if masked:  # padding, and a row of its own per position that drops whole tiles of keys
+        mask = (np.arange(S) < np.array([S, 200, 64, 1])[:, None])[:, None, None, :] & np.ones((B, 1, L, S), bool)
+        mask[0, 0, 7, :] = False
+        mask[0, 0, 7, 130] = True
+    got = ct.grouped_query_attention(ct.Tensor.from_numpy(q, ct.F32, GPU), gk, gv,
+                                     None if mask is None else ct.Tensor.from_numpy(mask, ct.BOOL, GPU)).numpy()
+    want = reference(q, k, v, mask)
+    bound = 2.0**-24 * (np.sqrt(D) + np.sqrt(S) + 8)
+    assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want)
+    rows = np.linalg.norm(got - want, axis=-1) / np.linalg.norm(want, axis=-1)
+    assert np.max(rows) <= 4 * bound
+
+
 @pytest.mark.parametrize("L,S,masked", [(5, 130, False), (5, 130, True), (1, 70, True), (70, 90, False)])
 @pytest.mark.parametrize("axis,start", [(0, 1), (1, 2), (2, 1), (3, 1)])
 def test_views_of_a_query_and_a_mask_are_read_through_their_strides(L, S, masked, axis, start):

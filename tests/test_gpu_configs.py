@@ -6,7 +6,7 @@ f32 K/V cache, through the C ABI.  (C1 and C2 run in test_gpu_parity.py.)
   C4  8B-width layers (d 4096, 32/8 heads, head dim 128, SwiGLU 14336, RoPE base 500000), batch 8 over 32768
       cached positions (bf16 opt-in): two full-width layers against the oracle, and the whole 32-layer model
       (weights drawn on the device) with the graph-replayed token loop equal to the eager one;
-  C5  1B bf16 decoder with unmerged LoRA (rank 16, alpha 32) on q and v: a 2 x 512 prefill (tiled matrix-core
+  C5  1B bf16 decoder with unmerged LoRA (rank 16, alpha 32) on q and v: a 2 x 512 prefill (staged matrix-core
       projections, matrix-core causal attention over the f32 cache) and decode steps against the oracle, and the
       full 4 x 4096 prefill in two chunks equal to one chunk.
 
@@ -135,7 +135,7 @@ C5 = oracle.ModelConfig(vocab=32000, layers=16, dimensions=2048, heads=32, kv_he
 
 
 def test_c5_1b_lora_prefill_2x512_and_decode_against_the_oracle():
-    say("case: C5 1B bf16 + LoRA r16 a32 on q/v, prefill 2 x 512 (tiled projections, matrix-core attention over the "
+    say("case: C5 1B bf16 + LoRA r16 a32 on q/v, prefill 2 x 512 (staged projections, matrix-core attention over the "
         "f32 cache), then 2 decode steps")
     ref, gpu = build_pair(C5, root=(5050, 0))
     B, P = 2, 512

@@ -1,6 +1,7 @@
 """Projections on the f32 matrix cores, against numpy in 64 bits and the CPU oracle: f32 weights over nine or more rows,
 and bf16 weights over 65 or more of the shapes whose activations are not split.  Edges of the work-group shapes, partial
-weight tiles, K remainders, every epilogue."""
+weight tiles, K remainders, every epilogue.  test_host_rules.py checks on the CPU that each shape takes the work-groups named
+beside it."""
 import numpy as np
 import pytest
 
@@ -16,10 +17,15 @@ GPU = ct.device("gpu")
 BOUND = 17 * 2.0**-24
 
 
-@pytest.mark.parametrize("rows,k,n", [(9, 4, 1), (16, 36, 130), (17, 1000, 333), (33, 688, 64), (65, 32, 2),
-                                      (129, 256, 8191), (700, 260, 2100), (2100, 64, 260)])
-def test_linear_f32_weights_over_many_rows(rows, k, n):
-    say(f"case: f32 linear {rows} x {k} -> {n}")
+# rows, k, n, work-group shape
+LINEAR_F32 = [(9, 4, 1, "32x16"), (16, 36, 130, "32x16"), (17, 1000, 333, "32x16"), (33, 688, 64, "32x16"),
+              (65, 32, 2, "32x16"), (129, 256, 8191, "64x32"), (700, 260, 2100, "64x32"), (2100, 64, 260, "64x32"),
+              (1030, 36, 2100, "64x64"), (2049, 36, 8200, "128x128")]
+
+
+@pytest.mark.parametrize("rows,k,n,shape", LINEAR_F32)
+def test_linear_f32_weights_over_many_rows(rows, k, n, shape):
+    say(f"case: f32 linear {rows} x {k} -> {n} ({shape})")
     rng = np.random.default_rng(rows)
     x, w, b = (rng.standard_normal(s).astype(np.float32) for s in ((rows, k), (n, k), (n,)))
     gx, gw, gb = (ct.Tensor.from_numpy(a, ct.F32, GPU) for a in (x, w, b))
@@ -40,10 +46,14 @@ def test_linear_f32_keeps_infinities_and_nans_to_their_rows():
     assert np.all(np.isfinite(np.delete(got, [3, 7], 0)))
 
 
-@pytest.mark.parametrize("rows,k,n", [(65, 64, 16), (65, 512, 17), (128, 256, 250), (129, 320, 48), (256, 64, 33),
-                                      (300, 4096, 1000), (300, 320, 8192), (1030, 64, 2100), (2049, 64, 8200)])
-def test_linear_bf16_weights_keep_whole_activations(rows, k, n):
-    say(f"case: bf16 linear {rows} x {k} -> {n}, f32 activations")
+LINEAR_BF16 = [(65, 64, 16, "32x16"), (65, 512, 17, "32x16"), (128, 256, 250, "32x16"), (129, 320, 48, "32x16"),
+               (256, 64, 33, "32x16"), (300, 4096, 1000, "32x16"), (300, 320, 8192, "64x64"), (700, 320, 2050, "64x32"),
+               (1030, 64, 2100, "64x64"), (2049, 64, 8200, "128x128")]
+
+
+@pytest.mark.parametrize("rows,k,n,shape", LINEAR_BF16)
+def test_linear_bf16_weights_keep_whole_activations(rows, k, n, shape):
+    say(f"case: bf16 linear {rows} x {k} -> {n}, f32 activations ({shape})")
     rng = np.random.default_rng(rows + n)
     x, w, b = (rng.standard_normal(s).astype(np.float32) for s in ((rows, k), (n, k), (n,)))
     bits, bias_bits = oracle.bf16_encode(w), oracle.bf16_encode(b)

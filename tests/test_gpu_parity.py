@@ -500,8 +500,9 @@ def test_streaming_decode_attention_over_many_keys(dimensions, heads, kv_heads, 
 
 
 @pytest.mark.parametrize("kv", ["f32", "bf16"])
+# 2 x 2048 rows: gate/up takes gemm_tiles, the other projections gemm_mid; so do two chunks of 1024 (see test_host_rules.py)
 def test_prefill_on_tiled_matrix_cores_with_lora_and_causal_attention(kv):
-    say(f"case: bf16 prefill B=2 x 2048, d=1024 (tiled projections + matrix-core causal attention), LoRA q/v, {kv} K/V")
+    say(f"case: bf16 prefill B=2 x 2048, d=1024 (staged projections + matrix-core causal attention), LoRA q/v, {kv} K/V")
     cfg = oracle.ModelConfig(vocab=512, layers=1, dimensions=1024, heads=16, kv_heads=4, hidden=2816, context=2056,
                              dtype="bf16", lora_rank=16, lora_alpha=32.0)
     weights = oracle.synthesize_weights(cfg, (61, 0), 0.03)
@@ -525,7 +526,7 @@ def test_prefill_on_tiled_matrix_cores_with_lora_and_causal_attention(kv):
     # K/V of an f32 cache) keep the gap to the oracle with the same K/V storage far below it
     assert np.max(np.abs(got - want)) <= 2e-2 and rel_err(got, near) <= 5e-4
     ids = want.argmax(-1).reshape(B, 1)
-    for step in range(2):  # decode over the 2048 keys the tiled QKV epilogue wrote
+    for step in range(2):  # decode over the 2048 keys the QKV epilogue wrote
         want = ref.logits(ids, rc)[:, -1]
         near = same.logits(ids, sc)[:, -1] if same is not ref else want
         got = gpu.logits(ids, gc)
@@ -537,7 +538,7 @@ def test_prefill_on_tiled_matrix_cores_with_lora_and_causal_attention(kv):
     gpu.logits(prompt[:, :1024], chunked_cache)
     chunked = gpu.logits(prompt[:, 1024:], chunked_cache)
     assert rel_err(chunked, full) <= 1e-4
-    # a truncated cache prefilled again from position 1500 (548 rows: the batched projection path, attention
+    # a truncated cache prefilled again from position 1500 (548 rows a sequence: all projections on gemm_mid, attention
     # with an offset) equals the single chunk
     chunked_cache.truncate(1500)
     again = gpu.logits(prompt[:, 1500:], chunked_cache)
@@ -545,10 +546,11 @@ def test_prefill_on_tiled_matrix_cores_with_lora_and_causal_attention(kv):
 
 
 def test_prefill_of_four_sequences_takes_the_tiled_projection_in_groups_of_four_row_blocks():
-    # 4 x 2048 rows are 32 row blocks of 256: each XCD takes a band of 4 and walks it in one group of 4 row blocks
-    # (the C5 order); two chunks of 1024 per sequence (16 row blocks, groups of 2) must give the same logits, and
-    # the 8 (sequence, KV head) pairs take the prefill attention's one-XCD-per-pair order
-    say("case: bf16 prefill B=4 x 2048, d=512, LoRA q/v, f32 K/V: tiled projections in groups of 4 row blocks")
+    # 4 x 2048 rows are 32 row blocks of 256: in gate/up (gemm_tiles; the narrower projections take gemm_mid) each XCD takes
+    # a band of 4 and walks it in one group of 4 row blocks (the C5 order); two chunks of 1024 per sequence (16 row blocks,
+    # groups of 2) must give the same logits, and the 8 (sequence, KV head) pairs take the prefill attention's
+    # one-XCD-per-pair order
+    say("case: bf16 prefill B=4 x 2048, d=512, LoRA q/v, f32 K/V: gate/up tiles in groups of 4 row blocks")
     cfg = oracle.ModelConfig(vocab=512, layers=1, dimensions=512, heads=8, kv_heads=2, hidden=1536, context=2056,
                              dtype="bf16", lora_rank=16, lora_alpha=32.0)
     ref, gpu = build_pair(cfg, root=(64, 0), scale=0.03)
@@ -560,7 +562,7 @@ def test_prefill_of_four_sequences_takes_the_tiled_projection_in_groups_of_four_
     say(f"  prefill logits: max|d| {np.max(np.abs(got - want)):.3g}, rel {rel_err(got, want):.3g}")
     assert np.max(np.abs(got - want)) <= 2e-2 and rel_err(got, want) <= 5e-4
     ids = want.argmax(-1).reshape(B, 1)
-    for step in range(2):  # decode over the keys the tiled QKV epilogue wrote
+    for step in range(2):  # decode over the keys the QKV epilogue wrote
         want = ref.logits(ids, rc)[:, -1]
         got = gpu.logits(ids, gc)
         assert np.max(np.abs(got - want)) <= 2e-2 and rel_err(got, want) <= 5e-4, step
@@ -613,10 +615,10 @@ def test_decode_with_lora_down_rows_folded_into_the_qkv_launch(rank, batch):
     assert np.array_equal(t1, t2) and np.array_equal(l1, l2)
 
 
-def test_tiled_prefill_with_lora_and_a_partial_qkv_column_block():
-    # d = 256, 8/2 heads of 32: the QKV projection has 24 weight tiles, one full column block of 16 and one of 8,
-    # which runs the tiled kernel's checked products and its LoRA epilogue on the missing tiles' slots
-    say("case: bf16 prefill B=2 x 512, d=256 (QKV 384 columns: a partial column block), LoRA q/v rank 16, f32 K/V")
+def test_staged_prefill_with_lora_and_a_qkv_of_three_column_blocks():
+    # d = 256, 8/2 heads of 32: the QKV projection has 24 weight tiles, three column blocks of gemm_mid, with its LoRA
+    # epilogue (a partial column block of gemm_tiles: test_gpu_layer_rows.py)
+    say("case: bf16 prefill B=2 x 512, d=256 (QKV 384 columns), LoRA q/v rank 16, f32 K/V")
     cfg = oracle.ModelConfig(vocab=256, layers=2, dimensions=256, heads=8, kv_heads=2, hidden=512, context=520,
                              dtype="bf16", lora_rank=16, lora_alpha=32.0)
     weights = oracle.synthesize_weights(cfg, (77, 0), 0.05)
@@ -636,7 +638,7 @@ def test_tiled_prefill_with_lora_and_a_partial_qkv_column_block():
     assert rel_err(without, want) >= 20 * 5e-4
     assert np.max(np.abs(got - want)) <= 2e-2 and rel_err(got, want) <= 5e-4
     ids = want.argmax(-1).reshape(B, 1)
-    for step in range(2):  # decode over the keys the tiled QKV epilogue wrote
+    for step in range(2):  # decode over the keys the QKV epilogue wrote
         want = ref.logits(ids, rc)[:, -1]
         got = gpu.logits(ids, gc)
         assert np.max(np.abs(got - want)) <= 2e-2 and rel_err(got, want) <= 5e-4, step

@@ -9,7 +9,7 @@ the graph-replayed token loop that bench.py times, over whole requests.
   C3  1B bf16, batch 32 over a 2048-position seeded prefix (the bf16 cache opt-in), 16 graph-replayed steps: the
       last logits and every id against the teacher-forced oracle, and the graph-replayed loop equal to the eager
       one bit for bit;
-  C5  1B bf16 with unmerged LoRA (rank 16, alpha 32) on q and v: a 1 x 4096 prefill (tiled matrix-core projections,
+  C5  1B bf16 with unmerged LoRA (rank 16, alpha 32) on q and v: a 1 x 4096 prefill (staged matrix-core projections,
       causal attention over the f32 cache) against the oracle's last-position logits, then 8 decode steps.
 
 Tolerance: bf16 logits within 2e-2 max-abs of the oracle; a generated id's oracle logit within 4e-2 of that

@@ -1,9 +1,14 @@
-"""What the host side decides for a call (attention key splits), without a GPU: the program
-tests/clients/host_checks.cpp calls the library's own functions."""
+"""What the host side decides for a call (kernels, attention key splits, workspaces, held device blocks), without a GPU:
+the program tests/clients/host_checks.cpp calls the library's own functions."""
 import os
 import subprocess
 
 import pytest
+
+import test_gpu_attention_rows
+import test_gpu_f32_rows
+import test_gpu_layer_rows
+import test_gpu_mid_rows
 
 PROGRAM = os.path.join(os.path.dirname(os.path.abspath(__file__)), "clients", "_build", "host_checks")
 
@@ -72,3 +77,66 @@ def test_many_rows_of_small_heads_are_not_split(head_dim, length, source, split_
     # 4 sequences, 32 / 8 heads: a wave per query row, so many rows fill the device without key splits and their merge
     splits, chunk = split(4, 32, 8, head_dim, False, length, source, False)
     assert (splits > 1) == split_up and splits * chunk >= source
+
+
+def test_freed_blocks_are_held_up_to_the_release_threshold():
+    # held; at threshold 0 the held one goes back at once and a freed one is not held; held again
+    assert checks("threshold").split() == ["1", "0", "0", "1"]
+
+
+def test_an_allocation_that_fails_is_tried_again_without_the_held_blocks():
+    assert checks("retry").split() == ["1", "1"]
+
+
+# ------------------------------------------------------------------------------------------ kernels of the GPU tests
+def projection(epilogue, rows, k, segments, bf16, bias=False, layer=False):
+    return checks("projection", epilogue, rows, k, *(list(segments) + [0, 0])[:3], bf16, bias, layer).strip()
+
+
+def layer_kernels(rows, d, heads, kv, hidden, bf16):
+    side = kv * d // heads
+    return [projection("qkv", rows, d, (d, side, side), bf16, layer=True),
+            projection("residual", rows, d, (d,), bf16, layer=True),
+            projection("swiglu", rows, d, (hidden, hidden), bf16, layer=True),
+            projection("residual", rows, hidden, (d,), bf16, layer=True)]
+
+
+def test_the_linear_tests_take_the_kernels_they_name():
+    for rows, k, n, bias, kernel in test_gpu_mid_rows.LINEAR:
+        assert projection("store", rows, k, (n,), True, bias) == kernel, (rows, k, n)
+    for rows, k, n, shape in test_gpu_f32_rows.LINEAR_F32:
+        assert projection("store", rows, k, (n,), False) == "f32 " + shape, (rows, k, n)
+    for rows, k, n, shape in test_gpu_f32_rows.LINEAR_BF16:
+        assert projection("store", rows, k, (n,), True) == "f32 " + shape, (rows, k, n)
+    named = {kernel for *_, kernel in test_gpu_mid_rows.LINEAR}
+    shapes = [{shape for *_, shape in table} for table in (test_gpu_f32_rows.LINEAR_F32, test_gpu_f32_rows.LINEAR_BF16)]
+    assert named == {"mid", "narrow", "tiles"} and shapes == [{"32x16", "64x32", "64x64", "128x128"}] * 2
+
+
+def test_the_layer_and_block_tests_take_the_kernels_they_name():
+    for batch, length, d, heads, kv, hidden, rank, dtype, kernels, _ in test_gpu_layer_rows.LAYERS:
+        assert layer_kernels(batch * length, d, heads, kv, hidden, dtype == "bf16") == kernels.split(", ")
+        if rank == 16:
+            assert projection("store", batch * length, d, (rank, rank), dtype == "bf16", layer=True) == "narrow"
+    for batch, length, d, heads, kv, hidden, rank, _, kernels in test_gpu_mid_rows.PROMPTS:
+        got = layer_kernels(batch * length, d, heads, kv, hidden, True)
+        assert [kernel.split()[0] for kernel in got] == kernels.split(", "), (batch, length, d, hidden)
+    for rows, hidden, kernels in test_gpu_mid_rows.SWIGLU:
+        got = [projection("swiglu", rows, 512, (hidden, hidden), True), projection("store", rows, hidden, (512,), True)]
+        assert [kernel.split()[0] for kernel in got] == kernels.split(", "), (rows, hidden)
+
+
+def test_the_attention_tests_take_the_kernel_they_name():
+    for B, H, KV, L, S, D, kernel in test_gpu_attention_rows.MANY:
+        for bf16 in (False, True):
+            for masked in (False, True):
+                assert checks("attention", B, H, KV, D, bf16, L, S, False, masked).strip() == kernel
+
+
+def test_the_prefill_parity_tests_take_the_kernels_they_name():
+    assert layer_kernels(2 * 2048, 1024, 16, 4, 2816, True) == ["mid", "mid", "tiles", "mid"]
+    assert layer_kernels(2 * 1024, 1024, 16, 4, 2816, True) == ["mid", "mid", "tiles", "mid"]
+    assert layer_kernels(2 * 548, 1024, 16, 4, 2816, True) == ["mid"] * 4
+    assert layer_kernels(4 * 2048, 512, 8, 2, 1536, True) == ["mid", "mid", "tiles", "mid"]
+    assert layer_kernels(2 * 512, 256, 8, 2, 512, True) == ["mid"] * 4
+    assert layer_kernels(4 * 4096, 2048, 32, 8, 5632, True) == ["tiles"] * 4
