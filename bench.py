@@ -1,17 +1,17 @@
 #!/usr/bin/env python3
-"""Decode throughput of the MI355X decoder token loop (BASELINE metric: decode tok/s, 1B bf16, b=1 and b=32,
+"""Decode throughput of the MI355X decoder token loop (decode tok/s, 1B bf16, b=1 and b=32,
 plus achieved HBM GB/s against the MI355X peak).
 
-Workload of `value` (BASELINE configs[1], "C2"): 1B-class GQA decoder (vocab 32000, d 2048, 16 layers, 32/8 heads,
+Workload of `value` ("C2"): 1B-class GQA decoder (vocab 32000, d 2048, 16 layers, 32/8 heads,
 head dim 64, SwiGLU 5632, RoPE base 10000), bf16 weights with f32 accumulation, batch 1, seeded N(0, 0.02) weights
 synthesised in HBM, a 128-token prompt of uniform random ids, greedy decode.  A step is one full token step on
 the GPU: embedding gather -> 16 fused layers -> final norm + LM head -> sampling -> id fed back, replayed from a
 HIP graph; exactly --steps steps are timed with HIP events on the library's compute stream after --warmup
 untimed steps.
 
-Also reported: the same C2 decode with temperature-1.0 sampling under an explicit key (configs[1]'s second leg),
-the b=32 decode over a 2048-token seeded K/V prefix (configs[2], "C3"), the 8B-class b=8 decode over
-a 32768-token seeded K/V prefix (configs[3], "C4"), the per-kernel roofline of
+Also reported: the same C2 decode with temperature-1.0 sampling under an explicit key,
+the b=32 decode over a 2048-token seeded K/V prefix ("C3"), the 8B-class b=8 decode over
+a 32768-token seeded K/V prefix ("C4"), the per-kernel roofline of
 the dominant kernel (gate/up projection: each layer's launch repeated back to back between two HIP events on the
 compute stream), a streaming-copy bandwidth reference, and the CPU oracle timed on this host (single thread) on
 a bounded sample of the same workload.
@@ -118,7 +118,7 @@ def decode_b1(ct, steps, warmup):
     prompt = np.random.default_rng(7).integers(0, C2["vocab"], size=(1, 128), dtype=np.int64)
     cache = ct.DecoderCache(decoder)
     ms, tokens = lm.benchmark(prompt, cache, warmup, steps, 0.0, (0, 0), True)
-    # the same decode with temperature-1.0 explicit-key sampling (BASELINE's second C2 leg), on a fresh cache
+    # the same decode with temperature-1.0 explicit-key sampling (C2's second leg), on a fresh cache
     scache = ct.DecoderCache(decoder)
     sampled_ms, _ = lm.benchmark(prompt, scache, warmup, steps, 1.0, SAMPLE_KEY, True)
     del scache
@@ -137,7 +137,7 @@ def decode_b1(ct, steps, warmup):
 
 def decode_b32(ct, steps, warmup, prefix=2048):
     """C3: batch 32, each sequence holding `prefix` cached tokens of seeded random K/V in the bf16 cache opt-in
-    (the KV-bandwidth regime BASELINE sizes in bf16)."""
+    (the KV-bandwidth regime, sized in bf16)."""
     B = 32
     decoder, lm = build_model(ct, C2, prefix + 3 + warmup + steps + 8, kv_dtype=ct.BF16)
     cache = ct.DecoderCache(decoder)

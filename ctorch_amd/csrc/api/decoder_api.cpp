@@ -5,7 +5,6 @@
 
 #include <algorithm>
 #include <cmath>
-
 #include <numeric>
 #include <stdexcept>
 
@@ -143,8 +142,9 @@ dl_status dl_grouped_query_attention_noalloc(const float* query, const void* key
         p.out = output;
         p.ldo = heads * D;
         if (p.splits > 1) {
-            // every split writes its (max, sum) pair and, when it holds keys, its partial output row; the merge
-            // skips splits without keys, so nothing has to start at zero
+            // every split writes its (max, sum) pair, and its partial output row when it holds keys (attention_rows and
+            // the small heads' kernel: always, zeros without); the merge takes no row that was not written, so nothing
+            // has to start at zero
             p.partial_o = scratch;
             p.partial_ml = scratch + rows * p.splits * D;
         }

@@ -36,7 +36,9 @@ typedef f32x2 f32x2_any __attribute__((aligned(4)));
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / kWave;
 constexpr int kBN = 128, kBM = 128;          // weight rows x activation rows per work-group
-/// Fewest rows: gemm_rows takes up to 64 in one launch (65 rows of 2048 -> 2048: 21.8 us in two, 18.3 here).
+/// Fewest rows: gemm_rows takes up to 64 in one launch (65 rows of 2048 -> 2048: 21.8 us in two, 18.3 here; the token loop
+/// over 65 sequences, whose repacked weights gemm_rows reads and this kernel does not, 36.0 -> 29.2 ms for 16 steps at 1B
+/// widths, over 256 95.1 -> 42.7; four 8B layers over 65 19.6 -> 15.3, over 256 40.9 -> 27.0).
 constexpr int kMinRows = gemm::kMaxRows + 1;
 constexpr int kStages = 3;                   // k pairs in LDS
 constexpr int kWeightBytes = kBN * 128;      // one k pair of weight fragments

@@ -1,7 +1,7 @@
 """ctypes bindings for the CPU oracle (liboracle.so) — TEST INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s ``cpu_baseline`` leg import this
-package, and only as the checker.  The product (``ctorch_amd``) never imports it.
+package, and only as the reference of checks.  The product (``ctorch_amd``) never imports it.
 
 Besides the raw bindings this module holds the harness's synthetic-model definition: the LM
 wrapper's parameter order (embedding ``tokens``, ``decoder.layer{i}...``, ``decoder.normalization``,

@@ -1,7 +1,7 @@
 /*
  * CPU oracle for the Ctorch decoder token loop — TEST INFRASTRUCTURE ONLY.
  * Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg load it,
- * and only as the checker.  See oracle.h for the parity pins.
+ * and only as the reference of checks.  See oracle.h for the parity pins.
  *
  * Restates the reference CPU arithmetic (paths relative to the reference tree):
  * f32 dot products sequential in k, RMSNorm statistics in double, the CPU

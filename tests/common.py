@@ -1,4 +1,4 @@
-"""Shared test helpers: one seeded model evaluated by the CPU oracle (the checker) and by the GPU library.
+"""Shared test helpers: one seeded model evaluated by the CPU oracle and by the GPU library.
 
 The oracle's synthetic weights (tests' and bench's common definition, oracle.synthesize_weights) are loaded
 into the library's modules through the C ABI: Embedding from tokens.weight, TransformerDecoder from the

@@ -1,8 +1,8 @@
-"""GPU parity at the full shapes of BASELINE's configs C3, C4 and C5, against the CPU oracle with the reference's
+"""GPU parity at the full shapes of the workloads C3, C4 and C5, against the CPU oracle with the reference's
 f32 K/V cache, through the C ABI.  (C1 and C2 run in test_gpu_parity.py.)
 
   C3  1B bf16 decoder, batch 32, each sequence holding 2048 cached positions of seeded random K/V (the bf16 cache
-      opt-in, as BASELINE sizes this regime), 2 decode steps;
+      opt-in), 2 decode steps;
   C4  8B-width layers (d 4096, 32/8 heads, head dim 128, SwiGLU 14336, RoPE base 500000), batch 8 over 32768
       cached positions (bf16 opt-in): two full-width layers against the oracle, and the whole 32-layer model
       (weights drawn on the device) with the graph-replayed token loop equal to the eager one;

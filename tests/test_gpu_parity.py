@@ -1,6 +1,6 @@
 """GPU parity of the decoder token loop against the CPU oracle, through the C ABI.
 
-Tolerances (BASELINE north star):
+Tolerances:
   f32 configs   logits max|d| / max|ref| <= 1e-4 per compared tensor, greedy ids identical;
   bf16 configs  logits max-abs <= 2e-2 (bf16 weights, f32 accumulation), always against the oracle with the
                 reference's f32 K/V cache; the GPU keeps f32 K/V by default and bf16 K/V where a test

@@ -1,4 +1,4 @@
-"""GPU parity at BASELINE's full workload lengths, against the CPU oracle with the reference's f32 K/V cache, through
+"""GPU parity at the full workload lengths, against the CPU oracle with the reference's f32 K/V cache, through
 the C ABI.  The reference's decode loop (src/nn/decoder.cpp:121-142, driven by examples/decoder_generate.cpp:26-31)
 runs these lengths; the shorter checks of test_gpu_parity.py and test_gpu_configs.py pin every kernel, these pin
 the graph-replayed token loop that bench.py times, over whole requests.

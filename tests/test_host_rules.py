@@ -14,6 +14,9 @@ PROGRAM = os.path.join(os.path.dirname(os.path.abspath(__file__)), "clients", "_
 
 
 def checks(*arguments):
+    if not os.path.exists(PROGRAM):
+        import __graft_entry__
+        __graft_entry__.build()
     run = subprocess.run([PROGRAM, *(str(int(a) if isinstance(a, bool) else a) for a in arguments)],
                          capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, (arguments, run.returncode, run.stderr)

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle before it is trusted as the parity checker (CPU only).
+"""Pins the CPU oracle before parity is checked against it (CPU only).
 
 Each check is chosen so that a plausible restatement mistake (dropped term, wrong index, wrong
 rounding order, swapped operand) fails it: published known-answer vectors, closed forms evaluated
